@@ -251,47 +251,44 @@ __global__ __launch_bounds__(1024) void k_clock_advance(DevClock* c, const doubl
 // ------------------------------------------------------------ launchers
 // Launch plan.  Every workgroup of the march kernel carries the same work: one tile through a
 // segment of `seg` planes, plus the two halo planes zs-1 and ze its predictor also visits.  The
-// chip holds `resident` = blocks_per_cu x ncu workgroups at once, so a launch of nb workgroups
-// runs in ceil(nb / resident) rounds of (seg + 2) planes each.  The plan takes the segment
-// length (kMinSeg planes at least) with the fewest rounds x (seg + 2): e.g. 2D 2048^2 in FP64
-// (34 tiles, two resident single-wave workgroups per SIMD) gets 35-plane segments in one round
-// of 2006 workgroups, where 32-plane segments need 2176 workgroups and a second round for 6 %
-// of the work.  The split changes which workgroup computes a cell, not how: results do not
-// depend on it (the conserved totals, summed per workgroup, only change their summation order).
+// chip holds `resident` = blocks_per_cu x ncu workgroups at once; a launch runs in full rounds of
+// that many and one round with the rest.  A plane of a round with w waves on a SIMD costs
+// c(w) = w + 1/4 in units of a wave's issue time: the FP64 pipe is shared, but a single wave does
+// not fill it (measured on MI355X: dependent-free FP64 instructions issue every 6.4 cycles with one
+// wave, 5.3 with two, 4.95 with four; the 2D kernel takes 3.5 us per plane with one wave per SIMD
+// and 6.3 us with two, the 3D one 6.5 and 10.8).  The plan takes the segment length with the fewest
+// (full rounds x c(full) + c(last round)) x (seg + 2).  Checked against fixed lengths on MI355X:
+//   2D 2048^2 FP64: 35 planes in one round of 2006 workgroups 247-250 us, 24 planes 252, 34 planes
+//     (2074 workgroups, a second round for 1 % of the work) 335;
+//   2D 600^2 FP64: 6 planes with one wave per SIMD 36.4 us, 3 planes with two 38.4, 4 planes 43;
+//   3D 96^3 FP64: 10 planes 134 us, 20 planes (one wave per SIMD) 150, 5 planes 144;
+//   grids that leave the chip idle take short segments, down to one plane, since what counts there
+//   is a workgroup's serial chain: 2D 301 x 173 27.4 us with 4 planes, 17.3 with one; 3D 50 x 41 x 37
+//   44.4 us with 4, 32.8 with 2 (one wave per SIMD), 37.0 with 1 (two waves).
+// The split changes which workgroup computes a cell, not how: results do not depend on it (the
+// conserved totals, summed per workgroup, only change their summation order).
 MarchPlan plan_march(const GridDev& G, int nd, int blocks_per_cu, int ncu)
 {
     MarchPlan P{};
     int const nm = G.n[nd - 1];
-    if (nd == 1) {  // one segment per thread: the same cost model over NT-segment workgroups
-        using S = MarchShape<1>;
-        P.L.ntile[0] = 1;
-        P.L.ntile[1] = 1;
-        int64_t const resident = (int64_t)std::max(blocks_per_cu, 1) * std::max(ncu, 1);
-        int64_t best_cost = -1;
-        for (int seg = std::min(4, nm); seg <= std::min(std::max(nm, 1), 1 << 16); ++seg) {
-            int64_t const nb = ((nm + seg - 1) / seg + S::NT - 1) / S::NT;
-            int64_t const cost = ((nb + resident - 1) / resident) * (seg + 2);
-            if (best_cost < 0 || cost < best_cost) {
-                best_cost = cost;
-                P.L.seglen = seg;
-                P.nb = nb;
-            }
-        }
-        return P;
-    }
-    int const HX = nd == 2 ? MarchShape<2>::HX : MarchShape<3>::HX;
-    int const HY = nd == 2 ? MarchShape<2>::HY : MarchShape<3>::HY;
-    int const TX = HX - 2;
-    int const TY = (nd == 3) ? HY - 2 : 1;
-    P.L.ntile[0] = (G.n[0] + TX - 1) / TX;
-    P.L.ntile[1] = (nd == 3) ? (G.n[1] + TY - 1) / TY : 1;
+    int const TX = nd == 1 ? 1 : (nd == 2 ? MarchShape<2>::HX : MarchShape<3>::HX) - 2;
+    int const TY = nd == 3 ? MarchShape<3>::HY - 2 : 1;
+    P.L.ntile[0] = nd == 1 ? 1 : (G.n[0] + TX - 1) / TX;
+    P.L.ntile[1] = nd == 3 ? (G.n[1] + TY - 1) / TY : 1;
     int64_t const tiles = (int64_t)P.L.ntile[0] * P.L.ntile[1];
-    int64_t const resident = (int64_t)std::max(blocks_per_cu, 1) * std::max(ncu, 1);
-    constexpr int kMinSeg = 4;
+    int64_t const cus = std::max(ncu, 1), per_cu = std::max(blocks_per_cu, 1);
+    int64_t const resident = per_cu * cus;
+    int const waves = (nd == 1 ? MarchShape<1>::NT : nd == 2 ? MarchShape<2>::NT : MarchShape<3>::NT) / 64;
+    auto plane_cost = [&](int64_t blocks) -> int64_t {  // 4 c(w) with `blocks` workgroups spread over the chip
+        int64_t const w = ((blocks + cus - 1) / cus * waves + 3) / 4;  // four SIMDs per CU
+        return w > 0 ? 4 * w + 1 : 0;
+    };
     int64_t best_cost = -1;
-    for (int seg = std::min(kMinSeg, nm); seg <= nm; ++seg) {
-        int64_t const nb = tiles * ((nm + seg - 1) / seg);
-        int64_t const cost = ((nb + resident - 1) / resident) * (seg + 2);
+    for (int seg = std::min(1, nm); seg <= std::min(nm, 1 << 16); ++seg) {
+        int64_t const segs = (nm + seg - 1) / seg;
+        // 1D: a workgroup holds one segment per thread
+        int64_t const nb = nd == 1 ? (segs + MarchShape<1>::NT - 1) / MarchShape<1>::NT : tiles * segs;
+        int64_t const cost = (nb / resident * plane_cost(resident) + plane_cost(nb % resident)) * (seg + 2);
         if (best_cost < 0 || cost < best_cost) {
             best_cost = cost;
             P.L.seglen = seg;
