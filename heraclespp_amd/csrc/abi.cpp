@@ -267,9 +267,7 @@ int hclpp_ctx_create(const hclpp_config* cfg, hclpp_ctx** out)
     for (int d = 0; d < 3; ++d) G.g[d] = cfg->g[d];
     // internal-mass gravity is a radial table like the point-mass one, rebuilt from rho every step
     G.gravity = cfg->gravity == HCLPP_GRAV_UNIFORM ? kUniformGravity : kPointMassGravity;
-    c->eos.gamma = cfg->gamma;
-    c->eos.gamma_m1 = cfg->gamma - 1;  // perfect_gas.cpp:13
-    c->eos.mmw = cfg->mmw;
+    c->eos = PerfectGas::make(cfg->gamma, cfg->mmw);
     c->eos32.gamma = (float)cfg->gamma;
     c->eos32.inv_gamma_m1 = (float)(1.0 / (cfg->gamma - 1));
     c->eos32.gamma_m1 = cfg->gamma - 1;
@@ -281,7 +279,7 @@ int hclpp_ctx_create(const hclpp_config* cfg, hclpp_ctx** out)
 
     // host tables (mesh/grid.cpp:31-44, :134-155; geometry.cpp trigonometry; gravity.cpp:44-55)
     std::vector<double> h;
-    size_t off_x[3], off_dx[3], off_xc[3];
+    size_t off_x[3], off_dx[3], off_xc[3], off_rdx[3], off_hc[3];
     for (int d = 0; d < 3; ++d) {
         int const nn = G.nwg[d];
         off_x[d] = h.size();
@@ -290,6 +288,14 @@ int hclpp_ctx_create(const hclpp_config* cfg, hclpp_ctx** out)
         for (int i = 0; i < nn; ++i) h.push_back(cfg->x[d][i + 1] - cfg->x[d][i]);
         off_xc[d] = h.size();
         for (int i = 0; i < nn; ++i) h.push_back((cfg->x[d][i] + cfg->x[d][i + 1]) / 2);
+        off_rdx[d] = h.size();
+        for (int i = 0; i < nn; ++i) h.push_back(1 / h[off_dx[d] + i]);
+        off_hc[d] = h.size();
+        for (int i = 0; i < nn; ++i) {
+            double const dist = (h[off_dx[d] + i] + h[off_dx[d] + std::min(i + 1, nn - 1)]) * 0.5;
+            h.push_back(dist);
+            h.push_back(1 / dist);
+        }
     }
     int const n1 = G.nwg[1];
     double const* x1 = cfg->x[1];
@@ -328,6 +334,8 @@ int hclpp_ctx_create(const hclpp_config* cfg, hclpp_ctx** out)
         G.x[d] = c->tables + off_x[d];
         G.dx[d] = c->tables + off_dx[d];
         G.xc[d] = c->tables + off_xc[d];
+        G.rdx[d] = c->tables + off_rdx[d];
+        G.hc[d] = c->tables + off_hc[d];
     }
     G.dcos = c->tables + off_dcos;
     G.sin_node = c->tables + off_sin;

@@ -26,6 +26,8 @@ struct GridDev {
     const double* x[3];       // node coordinates, nwg[d] + 1 entries
     const double* dx[3];      // cell sizes, nwg[d]
     const double* xc[3];      // cell centers, nwg[d]
+    const double* rdx[3];     // 1 / dx[d][i], nwg[d]
+    const double* hc[3];      // pairs (h, 1 / h) of the center distances h = (dx[d][i] + dx[d][i+1]) / 2, nwg[d] (the last: dx itself)
     const double* dcos;       // cos(x1[j]) - cos(x1[j+1]), nwg[1]
     const double* sin_node;   // sin(x1[j]), nwg[1] + 1
     const double* cot_mid;    // cos(m)/sin(m), m = (x1[j] + x1[j+1]) / 2, nwg[1]
@@ -93,6 +95,12 @@ __host__ __device__ __forceinline__ double face_area(const GridDev& G, int dir, 
     }
 }
 
+// Whether gravity acts along `dir` at all: the same for every cell, so a wave-uniform branch.
+__host__ __device__ __forceinline__ bool gravity_acts(const GridDev& G, int dir)
+{
+    return G.gravity == kUniformGravity ? G.g[dir] != 0 : dir == 0;
+}
+
 // hydro/time_step.hpp:61-76: the cell's CFL rate sum_d (|u_d| + c) / dx_geom_d
 template <int ND, int GEOM>
 __device__ __forceinline__ double cfl_rate(const GridDev& G, int i, int j, int k, const double* u, double c)
@@ -105,9 +113,13 @@ __device__ __forceinline__ double cfl_rate(const GridDev& G, int i, int j, int k
             dxg[2] *= G.xc[0][i] * G.sin_center[j];
         }
     }
+    int const idx[3] = {i, j, k};
     double rate = 0;
 #pragma unroll
-    for (int d = 0; d < ND; ++d) rate += fdiv(fabs(u[d]) + c, dxg[d]);
+    for (int d = 0; d < ND; ++d) {
+        if (GEOM == kCartesian || d == 0) rate += quot(fabs(u[d]) + c, dxg[d], G.rdx[d][idx[d]]);
+        else rate += fdiv(fabs(u[d]) + c, dxg[d]);
+    }
     return rate;
 }
 

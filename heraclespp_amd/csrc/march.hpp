@@ -13,9 +13,8 @@
 //    states to conservative form and applies the Hancock half step -- the
 //    reference's face_reconstruction / conv_prim_to_cons / Hancock kernels for
 //    one cell, in registers.
-//  * In-plane faces: each column publishes its right face state in LDS, the
-//    right neighbour solves the Riemann problem once per face, fluxes are
-//    exchanged back through LDS.  March-dim faces: the right face state of
+//  * In-plane faces: the right neighbour solves the Riemann problem once per
+//    face; x face states and fluxes pass between lanes, y ones through LDS.  March-dim faces: the right face state of
 //    plane h-1 is kept in registers and paired with plane h's left state.
 //  * The Godunov update of a cell accumulates dims in the reference order
 //    (flux, geometric sources, gravity per dim, march dim last), so with the
@@ -115,8 +114,11 @@ template <int ND, int GEOM, class Eos>
 __device__ __forceinline__ double state_rate(const GridDev& G, const Eos& eos, int i, int j, int k, const State<ND, typename Eos::real>& c)
 {
     if constexpr (kFp64State<Eos>) {
-        State<ND> const p = cons_to_prim(c, eos);
-        return cfl_rate<ND, GEOM>(G, i, j, k, &p.q[1], eos.sound(p[0], p[ND + 1]));
+        double evol, y, cs;
+        State<ND> const p = cons_to_prim_ey(c, eos, evol, y);
+        if constexpr (std::is_same_v<Eos, PerfectGas>) cs = eos.sound(p[0], p[ND + 1], y);
+        else cs = eos.sound(p[0], p[ND + 1]);
+        return cfl_rate<ND, GEOM>(G, i, j, k, &p.q[1], cs);
     } else {
         double const rho = c[0];
         double u[ND];
@@ -135,27 +137,37 @@ __device__ __forceinline__ double state_eint(const Eos& eos, const State<ND, typ
     else return eos.internal_energy_fp64(c);
 }
 
+// The distances of a cell's center to its neighbours' along one dim, with their reciprocals
+// (GridDev::hc): (dx[i-1] + dx[i]) / 2 and (dx[i] + dx[i+1]) / 2.
+struct CenterDist {
+    double hm, ym, hp, yp;
+};
+__device__ __forceinline__ CenterDist center_dist(const GridDev& G, int dim, int i)
+{
+    double const* h = G.hc[dim] + 2 * (i - 1);
+    return {h[0], h[1], h[2], h[3]};
+}
+
 // limited_linear_reconstruction.hpp:53-62 for one variable along one dim
 template <int LIM, class Eos, class T>
-__device__ __forceinline__ void reconstruct(T vm, T v, T vp, T dlm, T dl, T dlp, T& lo, T& hi)
+__device__ __forceinline__ void reconstruct(T vm, T v, T vp, const CenterDist& h, T dl, T& lo, T& hi)
 {
-    T const slope = slope_limiter<LIM, Eos, T>(Eos::div(vp - v, (dl + dlp) * T(0.5)), Eos::div(v - vm, (dlm + dl) * T(0.5)));
+    T const slope = slope_limiter<LIM, Eos, T>(Eos::quot_grid(vp - v, h.hp, h.yp), Eos::quot_grid(v - vm, h.hm, h.ym));
     lo = v - ((dl * T(0.5)) * slope);
     hi = v + ((dl * T(0.5)) * slope);
 }
 
 // Spherical sources of one dim for the cell's own face states (godunov_scheme.hpp:165-256),
-// applied to the accumulator in the reference order.
+// applied to the accumulator in the reference order.  pL and pR are the primitives of those
+// states, which the Riemann solves of the two faces have formed.
 template <class Eos, int ND, int GEOM>
-__device__ __forceinline__ void godunov_sources(const GridDev& G, const Eos& eos, int dim, int i, int j, typename Eos::real dtodv,
-                                                typename Eos::real dS, typename Eos::real dSp, const State<ND, typename Eos::real>& vL,
-                                                const State<ND, typename Eos::real>& vR, State<ND, typename Eos::real>& un)
+__device__ __forceinline__ void godunov_sources(const GridDev& G, int dim, int i, int j, typename Eos::real dtodv,
+                                                typename Eos::real dS, typename Eos::real dSp, const State<ND, typename Eos::real>& pL,
+                                                const State<ND, typename Eos::real>& pR, State<ND, typename Eos::real>& un)
 {
     using T = typename Eos::real;
     if constexpr (GEOM == kSpherical) {
         if (dim > 1) return;
-        State<ND, T> const pL = cons_to_prim(vL, eos);
-        State<ND, T> const pR = cons_to_prim(vR, eos);
         T const x0 = T(G.x[0][i]), x0p = T(G.x[0][i + 1]);
         if (dim == 0) {
             un[1] += src_pressure<Eos>(dtodv, pL[ND + 1], pR[ND + 1], dS, dSp);
@@ -213,15 +225,14 @@ __device__ __forceinline__ void predict_faces(const GridDev& G, const Eos& eos, 
 #pragma unroll
     for (int dim = 0; dim < ND; ++dim) {
         T const dl = T(G.dx[dim][idx[dim]]);
-        T const dlm = T(G.dx[dim][idx[dim] - 1]);
-        T const dlp = T(G.dx[dim][idx[dim] + 1]);
+        CenterDist const h = center_dist(G, dim, idx[dim]);
 #pragma unroll
         for (int v = 0; v < NV; ++v)
-            reconstruct<LIM, Eos>(nb[dim][0][v], p[v], nb[dim][1][v], dlm, dl, dlp, fp[0][dim][v], fp[1][dim][v]);
+            reconstruct<LIM, Eos>(nb[dim][0][v], p[v], nb[dim][1][v], h, dl, fp[0][dim][v], fp[1][dim][v]);
         if constexpr (NFX > 0) {
 #pragma unroll
             for (int f = 0; f < NFX; ++f)
-                reconstruct<LIM, Eos>(xnb[dim][0].f[f], x.f[f], xnb[dim][1].f[f], dlm, dl, dlp, xo[0][dim].f[f], xo[1][dim].f[f]);
+                reconstruct<LIM, Eos>(xnb[dim][0].f[f], x.f[f], xnb[dim][1].f[f], h, dl, xo[0][dim].f[f], xo[1][dim].f[f]);
         }
     }
 #pragma unroll
@@ -287,14 +298,16 @@ __device__ __forceinline__ void predict_faces(const GridDev& G, const Eos& eos, 
                     }
                 }
         }
-        T const g = T(gravity(G, i, dim));
+        if (gravity_acts(G, dim)) {
+            T const g = T(gravity(G, i, dim));
 #pragma unroll
-        for (int pos = 0; pos < ND; ++pos)
+            for (int pos = 0; pos < ND; ++pos)
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                fs[s][pos][1 + dim] += dth * g * rho_old[s][pos];
-                fs[s][pos][ND + 1] += dth * g * mom_old[s][pos][dim];
-            }
+                for (int s = 0; s < 2; ++s) {
+                    fs[s][pos][1 + dim] += dth * g * rho_old[s][pos];
+                    fs[s][pos][ND + 1] += dth * g * mom_old[s][pos][dim];
+                }
+        }
         if constexpr (NFX > 0) {  // extrapolation_reconstruction.hpp:315-323
 #pragma unroll
             for (int f = 0; f < NFX; ++f) {
@@ -317,18 +330,6 @@ __device__ __forceinline__ void predict_faces(const GridDev& G, const Eos& eos, 
     }
 }
 
-// Safe stand-in for cells outside the array (never feeds a valid output).
-template <int ND, class T>
-__device__ __forceinline__ State<ND, T> dummy_state()
-{
-    State<ND, T> p;
-    p[0] = 1;
-#pragma unroll
-    for (int d = 0; d < ND; ++d) p[1 + d] = 0;
-    p[ND + 1] = 1;
-    return p;
-}
-
 // The columns of a march workgroup.  Workgroup b of nb owns a tile of columns (3D: HX x HY, 2D: a
 // row of HX, 1D: NT segments of one column) and a segment of planes of the march dim; thread tid
 // owns column (a, bb) (ghost-inclusive coordinates of the in-plane dims; a tile's first and last
@@ -336,11 +337,8 @@ __device__ __forceinline__ State<ND, T> dummy_state()
 // so halo re-reads hit that XCD's L2.
 struct MarchColumn {
     int hx, hy, ox, oy, a, bb, zs, ze;
-    bool in_block;      // the thread owns a column of the tile
-    bool col_in_array;  // the column exists in memory
-    bool hancock_ok;    // the column needs a predictor
-    bool out_col;       // the column holds output cells
-    bool seg_ok;        // the segment holds planes
+    bool out_col;  // the column holds output cells
+    bool seg_ok;   // the segment holds planes (1D: a thread may have none)
 };
 
 template <int ND, int HX, int HY, int NT>
@@ -365,45 +363,30 @@ __device__ __forceinline__ MarchColumn march_column(const GridDev& G, const Fuse
         c.ox = G.ngh[0] + tx * TX;
         c.oy = (ND == 3) ? G.ngh[1] + ty * TY : 0;
     }
-    c.in_block = (ND == 1) || tid < HX * HY;
     c.a = c.ox - 1 + c.hx;
     c.bb = (ND == 3) ? c.oy - 1 + c.hy : 0;
     int const ngm = G.ngh[MD], nm = G.n[MD];
     c.zs = ngm + seg * L.seglen;
     c.ze = min(c.zs + L.seglen, ngm + nm);
-    c.col_in_array = c.in_block;
-    c.hancock_ok = c.in_block;
-    c.out_col = c.in_block;
-    if constexpr (ND >= 2) {
-        c.col_in_array = c.col_in_array && c.a < G.nwg[0];
-        c.hancock_ok = c.hancock_ok && c.a <= G.ngh[0] + G.n[0];
-        c.out_col = c.out_col && c.hx >= 1 && c.hx <= TX && c.a < G.ngh[0] + G.n[0];
-    }
-    if constexpr (ND == 3) {
-        c.col_in_array = c.col_in_array && c.bb < G.nwg[1];
-        c.hancock_ok = c.hancock_ok && c.bb <= G.ngh[1] + G.n[1];
-        c.out_col = c.out_col && c.hy >= 1 && c.hy <= TY && c.bb < G.ngh[1] + G.n[1];
-    }
     c.seg_ok = c.zs < ngm + nm;
-    if constexpr (ND == 1) {
-        c.col_in_array = c.seg_ok;
-        c.hancock_ok = c.seg_ok;
-        c.out_col = c.seg_ok;
-    }
+    c.out_col = c.seg_ok;
+    if constexpr (ND >= 2) c.out_col = c.out_col && c.hx >= 1 && c.hx <= TX && c.a < G.ngh[0] + G.n[0];
+    if constexpr (ND == 3) c.out_col = c.out_col && c.hy >= 1 && c.hy <= TY && c.bb < G.ngh[1] + G.n[1];
     return c;
 }
 
 // Minimum waves per SIMD the register allocator must allow.  Measured on MI355X: the 3D
-// FP32-storage kernel gains 23 % at 3 waves (168 VGPRs); the 3D Cartesian FP64 kernel gains 30 %
-// at 2 waves (256 VGPRs, 44 B of spills per lane, with the LDS parking below; two workgroups
-// fit a CU's LDS); the spherical 3D FP64 kernel loses 14 % at 2 waves (224 B of spills) and the
-// 2D kernels lose when forced above their natural 2 or 4.
-template <class Eos, int ND, int GEOM>
+// FP32-storage kernel gains 23 % at 3 waves (168 VGPRs); the 3D FP64 kernels gain 30 % at 2 waves
+// (256 VGPRs, with the LDS parking below; two workgroups fit a CU's LDS): RT 256^3 runs without a
+// spill, spherical Sedov with 12 spilled registers at 7.6 Gcell/s against 5.7 at one wave.  With a
+// passive scalar the spherical FP64 kernel spills 79 registers there and loses a third.  The 2D
+// kernels lose when forced above their natural 2 or 4.
+template <class Eos, int ND, int GEOM, int NFX>
 constexpr int march_min_waves()
 {
     if constexpr (ND != 3) return 1;
     else if constexpr (!kFp64State<Eos>) return 3;
-    else return GEOM == kCartesian ? 2 : 1;
+    else return GEOM == kSpherical && NFX > 0 ? 1 : 2;
 }
 
 // Load the NFX passive scalars (mass fractions, layout [f][cell]) of one cell.
@@ -418,7 +401,7 @@ __device__ __forceinline__ Frac<NFX, S> load_frac(const StepArraysT<S>& A, const
 
 // NFX: passive scalars carried through the step (0, or 1 for the kernels of step_fused_fx.hip).
 template <class Eos, int ND, int GEOM, int RS, int LIM, int NFX, int HX, int HY, int NT>
-__global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM>())) void k_step_march(GridDev G, Eos eos, StepArraysT<typename Eos::real> A, FusedLayout L)
+__global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM, NFX>())) void k_step_march(GridDev G, Eos eos, StepArraysT<typename Eos::real> A, FusedLayout L)
 {
     using T = typename Eos::real;
     using X = Frac<NFX, T>;
@@ -432,23 +415,25 @@ __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM>())) void k_step
     constexpr int TY = (ND == 3) ? HY - 2 : 1;
     constexpr int NXCH = NP > 0 ? NP : 1;
     // Barriers per plane: one after the primitive plane (double-buffered by plane parity) and, in
-    // 3D, one after the y face states and one after the y fluxes, which have buffers of their own,
-    // so no write waits for the readers of the previous plane's buffer beyond the barrier that
-    // already separates them.  x faces are exchanged between lanes (lane_shift), not through LDS.
+    // 3D, one after the y face states and one after the y fluxes.  The y face states take the
+    // primitive buffer of the other parity (its plane is read out by then) and the fluxes a buffer
+    // of their own, so no write waits for the readers of the previous plane's buffer beyond the
+    // barrier that already separates them.  x faces are exchanged between lanes (lane_shift), not
+    // through LDS.
     __shared__ T s_prim[2][NL][PY][PX];
-    constexpr int NYB = ND == 3 ? 1 : 0;  // LDS exchange buffers (the y dim of a 3D tile)
-    __shared__ T s_st[NYB > 0 ? NYB : 1][NYB > 0 ? NL : 1][NYB > 0 ? HY : 1][NYB > 0 ? HX : 1];
-    __shared__ T s_fl[NYB > 0 ? NYB : 1][NYB > 0 ? NL : 1][NYB > 0 ? HY : 1][NYB > 0 ? HX : 1];
+    __shared__ T s_fl[ND == 3 ? NL : 1][ND == 3 ? HY : 1][ND == 3 ? HX : 1];
+    // 3D spherical: the primitives a column's right y face gets in its neighbour's Riemann solve
+    // (velocities along y and z, pressure), which the column's geometric sources read; forming them
+    // again costs a state conversion per face (Sedov 7.15 -> 7.4 Gcell/s without)
+    constexpr bool kFaceP = ND == 3 && GEOM == kSpherical;
+    __shared__ T s_fp[kFaceP ? NV - 2 : 1][kFaceP ? HY : 1][kFaceP ? HX : 1];
     __shared__ double s_red[NT / 64];
     // Per-thread parking of the values plane h-1 hands to plane h (its right march face state,
     // its partial update and its left march flux, and the scalar's): written at the end of a
     // plane, read back when plane h completes plane h-1.  Only the owning thread touches its
     // slots, so no barrier is involved, and the registers are free across the plane's
-    // arithmetic.  Used where it pays (measured): the 3D FP32-storage kernel, whose register
-    // budget is set for 3 waves per SIMD (spills go from 40-152 to 0-92 B per lane; RT 512^3
-    // +6 %, spherical Sedov +26 %), and the 3D Cartesian FP64 kernel run at 2 waves per SIMD.
-    // In spherical FP64 and in 2D it gained nothing or lost.
-    constexpr bool kPark = ND == 3 && (!kFp64State<Eos> || GEOM == kCartesian);
+    // arithmetic.  3D only: in 2D it gained nothing.
+    constexpr bool kPark = ND == 3 && !(NFX > 0 && kFp64State<Eos> && GEOM == kSpherical);
     constexpr int NPARK = kPark ? 3 * NV + 3 * NFX : 1;
     __shared__ T s_park[NPARK][kPark ? NT : 1];
 
@@ -461,9 +446,18 @@ __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM>())) void k_step
 
     int const tid = threadIdx.x;
     MarchColumn const mc = march_column<ND, HX, HY, NT>(G, L, blockIdx.x, gridDim.x, tid);
-    int const hx = mc.hx, hy = mc.hy, ox = mc.ox, oy = mc.oy, a = mc.a, bb = mc.bb, zs = mc.zs, ze = mc.ze;
-    bool const in_block = mc.in_block, col_in_array = mc.col_in_array, hancock_ok = mc.hancock_ok, out_col = mc.out_col;
-    bool const seg_ok = mc.seg_ok;
+    int const hx = mc.hx, hy = mc.hy, ox = mc.ox, oy = mc.oy, zs = mc.zs, ze = mc.ze;
+    bool const out_col = mc.out_col, seg_ok = mc.seg_ok;
+    // Columns of a ragged last tile that lie beyond the array repeat its last column, so every lane
+    // runs the same code on a valid state and no value is selected around it: only the columns that
+    // hold output cells store, reduce or are read by one that does.  (With a branch around each part
+    // that a column may not need the compiler kept a second, initialised copy of every result of it:
+    // 70 register moves per plane of the 3D kernel, 3 % of its time.)
+    int const a = ND >= 2 ? min(mc.a, G.nwg[0] - 1) : 0, bb = ND == 3 ? min(mc.bb, G.nwg[1] - 1) : 0;
+    // Waves of a 3D tile all of whose rows lie beyond the last row that needs a predictor (bb = ngh + n)
+    // only keep the barriers.
+    static_assert(ND == 1 || NT == HX * HY, "one thread per column of the tile");
+    bool const live = ND < 3 || oy - 1 + __builtin_amdgcn_readfirstlane(hy) <= G.ngh[1] + G.n[1];
 
     // ring cells of the primitive plane (in-plane distance 2 from the output tile)
     constexpr int NRING = (ND == 3) ? 2 * (PX - 2) + 2 * (PY - 2) : ((ND == 2) ? 2 : 0);
@@ -471,27 +465,21 @@ __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM>())) void k_step
     double r_inv = reduce_identity<kMax>();
     double r_emin = reduce_identity<kMin>();
     double r_sum[NV];
+    // 3D spherical FP64 (256 registers): four of the conserved totals live in LDS (the thread's own
+    // slots) instead of in registers across the march, as many as two workgroups per CU leave room
+    // for (Sedov 7.0 -> 7.4 Gcell/s)
+    constexpr int kSumLds = kPark && kFp64State<Eos> && GEOM == kSpherical && NFX == 0 ? 4 : 0;
+    __shared__ double s_sum[kSumLds > 0 ? kSumLds : 1][kSumLds > 0 ? NT : 1];
 #pragma unroll
-    for (int v = 0; v < NV; ++v) r_sum[v] = 0;
-
-    auto prim_at = [&](int ca, int cb, int m) -> State<ND, T> {
-        bool ok = m >= 0 && m < G.nwg[MD];
-        if constexpr (ND >= 2) ok = ok && ca >= 0 && ca < G.nwg[0];
-        if constexpr (ND == 3) ok = ok && cb >= 0 && cb < G.nwg[1];
-        if (!ok) return dummy_state<ND, T>();
-        return cons_to_prim(load_cons<ND>(A, G, cell_at<ND>(G, ca, cb, m)), eos);
-    };
-    auto frac_at = [&](int ca, int cb, int m) -> X {
-        bool ok = m >= 0 && m < G.nwg[MD];
-        if constexpr (ND >= 2) ok = ok && ca >= 0 && ca < G.nwg[0];
-        if constexpr (ND == 3) ok = ok && cb >= 0 && cb < G.nwg[1];
-        if (!ok) return zero_frac<NFX, T>();
-        return load_frac<NFX>(A, G, cell_at<ND>(G, ca, cb, m));
-    };
+    for (int v = 0; v < NV; ++v) {
+        if (v < kSumLds) s_sum[v][tid] = 0;
+        else r_sum[v] = 0;
+    }
 
     // ring cell of this thread (at most one: NRING <= NT), fixed for the whole march
     static_assert(NRING <= NT, "one ring cell per thread");
-    bool const has_ring = tid < NRING;
+    // 3D: the ring is the first wave's work (a scalar branch); 2D: of the wave's first two lanes
+    bool const has_ring = ND == 3 && NRING == 64 ? __builtin_amdgcn_readfirstlane(tid) < NRING : tid < NRING;
     int ring_px = 0, ring_py = 0;
     if constexpr (ND == 2) {
         ring_px = tid == 0 ? 0 : PX - 1;
@@ -502,20 +490,20 @@ __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM>())) void k_step
         else if (r < 2 * (PX - 2) + (PY - 2)) { ring_px = 0; ring_py = 1 + r - 2 * (PX - 2); }
         else { ring_px = PX - 1; ring_py = 1 + r - 2 * (PX - 2) - (PY - 2); }
     }
-    int const ring_a = ox - 2 + ring_px, ring_b = (ND == 3) ? oy - 2 + ring_py : 0;
-    bool ring_in = has_ring;
-    if constexpr (ND >= 2) ring_in = ring_in && ring_a >= 0 && ring_a < G.nwg[0];
-    if constexpr (ND == 3) ring_in = ring_in && ring_b >= 0 && ring_b < G.nwg[1];
+    int const ring_a = ND >= 2 ? min(ox - 2 + ring_px, G.nwg[0] - 1) : 0;
+    int const ring_b = ND == 3 ? min(oy - 2 + ring_py, G.nwg[1] - 1) : 0;
 
     // pipeline registers.  Global loads run one plane ahead of their use (own column: plane h+2
     // while plane h is processed; ring cell: plane h+1), so their latency hides behind a plane
-    // of arithmetic instead of stalling the workgroup at the LDS barrier.
+    // of arithmetic instead of stalling the workgroup at the LDS barrier.  In 3D they are issued
+    // after the predictor (kLate), whose face states need the registers more: the Riemann solves
+    // still cover the latency (RT 256^3 10.9 -> 11.3 Gcell/s, FP32 21.5 -> 22.0, Sedov 7.4 -> 7.6).
+    constexpr bool kLate = ND == 3;
     State<ND, T> pm, p0, pp, c0, cp, cnext, rnext;
-    // Carried from plane to plane where registers allow (measured): the internal energies of c0
-    // and cp that their pressure recovery forms, and dt / dV of plane h-1 for its completion.
-    // The 3D Cartesian FP64 kernel (2 waves per SIMD) and the 3D spherical FP32 one recompute
-    // them instead: the extra registers spill there.
-    constexpr bool kCarry = !(ND == 3 && (kFp64State<Eos> == (GEOM == kCartesian)));
+    // Carried from plane to plane: the internal energies of c0 and cp that their pressure recovery
+    // forms, and dt / dV of plane h-1 for its completion.  The 3D spherical kernels recompute them
+    // instead: there the extra registers spill (FP64 Sedov 7.0 -> 7.4 Gcell/s without, FP32 12.6 -> 13.1).
+    constexpr bool kCarry = !(ND == 3 && GEOM == kSpherical);
     double e0 = 1, ep = 1;
     T dtodv_prev = 0;
     State<ND, T> fsR_prev, Fm_prev, part_prev;  // in registers, or in s_park when kPark
@@ -534,36 +522,28 @@ __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM>())) void k_step
     X xfR_prev = xm, xpart_prev = xm, ffm_prev = xm;
     int const zfirst = seg_ok ? zs - 1 : 0;
     int const zlast = seg_ok ? ze : -1;
-    bool rnext_ok = false;
-    if (col_in_array) {
-        pm = prim_at(a, bb, zfirst - 1);
+    if (seg_ok) {
+        pm = cons_to_prim(load_cons<ND>(A, G, cell_at<ND>(G, a, bb, zfirst - 1)), eos);
         c0 = load_cons<ND>(A, G, cell_at<ND>(G, a, bb, zfirst));
         if constexpr (kCarry) p0 = cons_to_prim_e(c0, eos, e0);
         else p0 = cons_to_prim(c0, eos);
-        if (zfirst <= zlast) cnext = load_cons<ND>(A, G, cell_at<ND>(G, a, bb, zfirst + 1));
+        cnext = load_cons<ND>(A, G, cell_at<ND>(G, a, bb, zfirst + 1));
         if constexpr (NFX > 0) {
-            xm = frac_at(a, bb, zfirst - 1);
+            xm = load_frac<NFX>(A, G, cell_at<ND>(G, a, bb, zfirst - 1));
             x0 = load_frac<NFX>(A, G, cell_at<ND>(G, a, bb, zfirst));
-            if (zfirst <= zlast) xnext = load_frac<NFX>(A, G, cell_at<ND>(G, a, bb, zfirst + 1));
+            xnext = load_frac<NFX>(A, G, cell_at<ND>(G, a, bb, zfirst + 1));
         }
-    } else {
-        pm = dummy_state<ND, T>();
-        p0 = dummy_state<ND, T>();
-        c0 = dummy_state<ND, T>();
     }
     if constexpr (ND >= 2) {
-        rnext_ok = ring_in && zfirst >= 0 && zfirst < G.nwg[MD] && zfirst <= zlast;
-        if (rnext_ok) {
+        if (has_ring) {
             rnext = load_cons<ND>(A, G, cell_at<ND>(G, ring_a, ring_b, zfirst));
             if constexpr (NFX > 0) rxnext = load_frac<NFX>(A, G, cell_at<ND>(G, ring_a, ring_b, zfirst));
         }
     }
 
     if constexpr (kPark) {  // plane zfirst-1's primitives of the own column, where the loop reads them
-        if (in_block) {
 #pragma unroll
-            for (int v = 0; v < NV; ++v) s_prim[(zfirst - 1) & 1][v][(ND == 3) ? hy + 1 : 0][hx + 1] = pm[v];
-        }
+        for (int v = 0; v < NV; ++v) s_prim[(zfirst - 1) & 1][v][(ND == 3) ? hy + 1 : 0][hx + 1] = pm[v];
     }
     auto park = [&](int slot, T v) {
         if constexpr (kPark) s_park[slot][tid] = v;
@@ -573,46 +553,41 @@ __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM>())) void k_step
         else return T(0);
     };
 
+    auto prefetch_column = [&](int h) {
+        if (h < zlast) {
+            cnext = load_cons<ND>(A, G, cell_at<ND>(G, a, bb, h + 2));
+            if constexpr (NFX > 0) xnext = load_frac<NFX>(A, G, cell_at<ND>(G, a, bb, h + 2));
+        }
+    };
+    auto prefetch_ring = [&](int h) {
+        if (h < zlast) {
+            rnext = load_cons<ND>(A, G, cell_at<ND>(G, ring_a, ring_b, h + 1));
+            if constexpr (NFX > 0) rxnext = load_frac<NFX>(A, G, cell_at<ND>(G, ring_a, ring_b, h + 1));
+        }
+    };
+
     for (int h = zfirst; h <= zlast; ++h) {
         int const pb = h & 1;
         // ---- plane h+1 of this column (prefetched), and the prefetch of plane h+2
-        if (col_in_array) {
-            cp = cnext;
-            xp = xnext;
-            if (h + 1 <= zlast) {
-                cnext = load_cons<ND>(A, G, cell_at<ND>(G, a, bb, h + 2));
-                if constexpr (NFX > 0) xnext = load_frac<NFX>(A, G, cell_at<ND>(G, a, bb, h + 2));
-            }
-            if constexpr (kCarry) pp = cons_to_prim_e(cp, eos, ep);
-            else pp = cons_to_prim(cp, eos);
-        } else {
-            cp = dummy_state<ND, T>();
-            pp = dummy_state<ND, T>();
-        }
+        cp = cnext;
+        xp = xnext;
+        if constexpr (!kLate) prefetch_column(h);
+        if constexpr (kCarry) pp = cons_to_prim_e(cp, eos, ep);
+        else pp = cons_to_prim(cp, eos);
         // ---- plane h primitives in LDS (own column + ring)
         if constexpr (ND >= 2) {
-            State<ND, T> ring_c;
-            X const rx = rnext_ok ? rxnext : zero_frac<NFX, T>();
-            bool const ring_ok = rnext_ok;
-            if (ring_ok) ring_c = rnext;
-            rnext_ok = ring_in && h + 1 < G.nwg[MD] && h + 1 <= zlast;
-            if (rnext_ok) {
-                rnext = load_cons<ND>(A, G, cell_at<ND>(G, ring_a, ring_b, h + 1));
-                if constexpr (NFX > 0) rxnext = load_frac<NFX>(A, G, cell_at<ND>(G, ring_a, ring_b, h + 1));
-            }
-            State<ND, T> const pr = ring_ok ? cons_to_prim(ring_c, eos) : dummy_state<ND, T>();
             // buffer h & 1 was last read at plane h - 2, before the barrier of plane h - 1
-            if (in_block) {
 #pragma unroll
-                for (int v = 0; v < NV; ++v) s_prim[pb][v][(ND == 3) ? hy + 1 : 0][hx + 1] = p0[v];
+            for (int v = 0; v < NV; ++v) s_prim[pb][v][(ND == 3) ? hy + 1 : 0][hx + 1] = p0[v];
 #pragma unroll
-                for (int f = 0; f < NFX; ++f) s_prim[pb][NV + f][(ND == 3) ? hy + 1 : 0][hx + 1] = x0.f[f];
-            }
+            for (int f = 0; f < NFX; ++f) s_prim[pb][NV + f][(ND == 3) ? hy + 1 : 0][hx + 1] = x0.f[f];
             if (has_ring) {
+                State<ND, T> const pr = cons_to_prim(rnext, eos);
 #pragma unroll
                 for (int v = 0; v < NV; ++v) s_prim[pb][v][ring_py][ring_px] = pr[v];
 #pragma unroll
-                for (int f = 0; f < NFX; ++f) s_prim[pb][NV + f][ring_py][ring_px] = rx.f[f];
+                for (int f = 0; f < NFX; ++f) s_prim[pb][NV + f][ring_py][ring_px] = rxnext.f[f];
+                if constexpr (!kLate) prefetch_ring(h);
             }
             __syncthreads();
         }
@@ -624,7 +599,7 @@ __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM>())) void k_step
         State<ND, T> fs[2][ND];
         X xf[2][ND];
         double qv = 0;
-        if (hancock_ok) {
+        if (live) {
             State<ND, T> nb3[ND][2];
             X xnb[ND][2];
             if constexpr (ND >= 2) {
@@ -676,11 +651,15 @@ __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM>())) void k_step
             for (int s = 0; s < 2; ++s)
 #pragma unroll
                 for (int d = 0; d < ND; ++d) {
-                    fs[s][d] = c0;
+                    fs[s][d] = p0;
                     xf[s][d] = x0;
                 }
         }
 
+        if constexpr (kLate) {
+            prefetch_column(h);
+            if (has_ring) prefetch_ring(h);
+        }
         // ---- in-plane fluxes and the in-plane part of the update of plane h
         State<ND, T> part = c0;
         T old_rho = c0[0], old_mom = c0[1 + MD], src_m = 0;
@@ -688,9 +667,9 @@ __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM>())) void k_step
 #pragma unroll
         for (int f = 0; f < NFX; ++f) xpart.f[f] = x0.f[f] * c0[0];
         T dtodv = 0;
-        if (out_plane) {
+        if (out_plane && live) {
+            dtodv = kCarry ? T(qv) : T(fdiv(dt_d, cell_volume<ND, GEOM>(G, ci, cj, ck)));
             if (out_col) {
-                dtodv = kCarry ? T(qv) : T(fdiv(dt_d, cell_volume<ND, GEOM>(G, ci, cj, ck)));
                 // min internal energy of the consumed state (internal_energy.cpp:25-40), as its
                 // pressure recovery formed it
                 r_emin = reduce_combine<kMin>(r_emin, kCarry ? e0 : state_eint<ND>(eos, c0));
@@ -701,95 +680,108 @@ __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM>())) void k_step
                     }
                 }
             }
+        }
+        if (out_plane) {
             if constexpr (ND >= 2) {
                 // Riemann solve of the left face along in-plane dim p, given the right face state
-                // (and scalar face values) of the column on the left; a column that needs no
-                // such face yields its own state as a placeholder flux
-                auto solve = [&](int p, bool need, const State<ND, T>& left, const X& xleft, State<ND, T>& F, X& XF) {
-                    XF = zero_frac<NFX, T>();
-                    if (need) {
-                        F = riemann<RS>(left, fs[0][p], p, eos);
-                        // upwind face of the scalar (godunov_scheme.hpp:265-287): this cell's
-                        // left face when the mass flux is negative, else the left cell's right face
+                // (and scalar face values) of the column on the left; pl and pr are the primitives
+                // of its two sides
+                auto solve = [&](int p, const State<ND, T>& left, const X& xleft, State<ND, T>& F, X& XF, State<ND, T>& pl, State<ND, T>& pr) {
+                    FaceSide<ND, Eos> const L = face_side(left, eos), R = face_side(fs[0][p], eos);
+                    F = riemann<RS>(left, fs[0][p], L, R, p, eos);
+                    pl = L.p;
+                    pr = R.p;
+                    // upwind face of the scalar (godunov_scheme.hpp:265-287): this cell's
+                    // left face when the mass flux is negative, else the left cell's right face
 #pragma unroll
-                        for (int f = 0; f < NFX; ++f) XF.f[f] = (F[0] < 0 ? xf[0][p].f[f] : xleft.f[f]) * F[0];
-                    } else {
-                        F = c0;
-                    }
+                    for (int f = 0; f < NFX; ++f) XF.f[f] = (F[0] < 0 ? xf[0][p].f[f] : xleft.f[f]) * F[0];
                 };
                 // the update of dim p (flux, sources, gravity) in the reference order: dims in turn
-                auto accumulate = [&](int p, const State<ND, T>& FL, const State<ND, T>& FR, const X& XL, const X& XR) {
+                auto accumulate = [&](int p, const State<ND, T>& FL, const State<ND, T>& FR, const X& XL, const X& XR, const State<ND, T>& qL,
+                                      const State<ND, T>& qR) {
                     T const dS = T(face_area<ND, GEOM>(G, p, ci, cj, ck));
                     T const dSp = T(face_area<ND, GEOM>(G, p, ci + (p == 0), cj + (p == 1), ck));
 #pragma unroll
                     for (int v = 0; v < NV; ++v) part[v] += dtodv * ((FL[v] * dS) - (FR[v] * dSp));
-                    godunov_sources<Eos, ND, GEOM>(G, eos, p, ci, cj, dtodv, dS, dSp, fs[0][p], fs[1][p], part);
-                    T const g = T(gravity(G, ci, p));
-                    part[1 + p] += dt * g * c0[0];
-                    part[ND + 1] += dt * g * c0[1 + p];
+                    godunov_sources<Eos, ND, GEOM>(G, p, ci, cj, dtodv, dS, dSp, qL, qR, part);
+                    if (gravity_acts(G, p)) {
+                        T const g = T(gravity(G, ci, p));
+                        part[1 + p] += dt * g * c0[0];
+                        part[ND + 1] += dt * g * c0[1 + p];
+                    }
 #pragma unroll
                     for (int f = 0; f < NFX; ++f) xpart.f[f] += dtodv * ((XL.f[f] * dS) - (XR.f[f] * dSp));
                 };
-                // y (3D): right face states through LDS; s_st was last read before the flux
-                // barrier of the previous plane
-                if constexpr (ND == 3) {
-                    if (in_block) {
+                if (live) {
+                    // y (3D): right face states through LDS, in the columns' own slots of the other
+                    // primitive plane, whose values (plane h - 1) were last read before this point:
+                    // by other columns at plane h - 1, by this one (kPark) above
+                    if constexpr (ND == 3) {
 #pragma unroll
-                        for (int v = 0; v < NV; ++v) s_st[0][v][hy][hx] = fs[1][1][v];
+                        for (int v = 0; v < NV; ++v) s_prim[pb ^ 1][v][hy + 1][hx + 1] = fs[1][1][v];
 #pragma unroll
-                        for (int f = 0; f < NFX; ++f) s_st[0][NV + f][hy][hx] = xf[1][1].f[f];
+                        for (int f = 0; f < NFX; ++f) s_prim[pb ^ 1][NV + f][hy + 1][hx + 1] = xf[1][1].f[f];
                     }
-                }
-                {  // x: the column at x - 1 is the lane beside (every lane executes the shifts)
-                    State<ND, T> left;
-                    X xleft;
+                    // x: the column at x - 1 is the lane beside
+                    State<ND, T> left, FL, FR, pl, qL, qR;
+                    X xleft, XL, XR;
 #pragma unroll
                     for (int v = 0; v < NV; ++v) left[v] = lane_shift<HX, true>(fs[1][0][v]);
 #pragma unroll
                     for (int f = 0; f < NFX; ++f) xleft.f[f] = lane_shift<HX, true>(xf[1][0].f[f]);
-                    bool const need = hancock_ok && hx >= 1 && (ND == 2 || (hy >= 1 && hy <= TY));
-                    State<ND, T> FL, FR;
-                    X XL, XR;
-                    solve(0, need, left, xleft, FL, XL);
+                    solve(0, left, xleft, FL, XL, pl, qL);
                     // the right face's flux is the left flux of the column at x + 1
 #pragma unroll
                     for (int v = 0; v < NV; ++v) FR[v] = lane_shift<HX, false>(FL[v]);
 #pragma unroll
                     for (int f = 0; f < NFX; ++f) XR.f[f] = lane_shift<HX, false>(XL.f[f]);
-                    if (out_col) accumulate(0, FL, FR, XL, XR);
+                    if constexpr (GEOM == kSpherical) {  // the primitives of this column's own right face
+                        qR[0] = fs[1][0][0];
+#pragma unroll
+                        for (int v = 1; v < NV; ++v) qR[v] = lane_shift<HX, false>(pl[v]);
+                    }
+                    accumulate(0, FL, FR, XL, XR, qL, qR);
                 }
                 if constexpr (ND == 3) {  // y: left states and right fluxes through LDS
                     __syncthreads();
-                    bool const need = hancock_ok && hy >= 1 && hx >= 1 && hx <= TX;
-                    State<ND, T> left, FL, FR;
-                    X xleft = zero_frac<NFX, T>(), XL, XR;
-                    if (need) {
+                    State<ND, T> left, FL, FR, pl, qL, qR;
+                    X xleft, XL, XR;
+                    if (live) {
+                        int const hyl = max(hy - 1, 0);
 #pragma unroll
-                        for (int v = 0; v < NV; ++v) left[v] = s_st[0][v][hy - 1][hx];
+                        for (int v = 0; v < NV; ++v) left[v] = s_prim[pb ^ 1][v][hyl + 1][hx + 1];
 #pragma unroll
-                        for (int f = 0; f < NFX; ++f) xleft.f[f] = s_st[0][NV + f][hy - 1][hx];
-                    }
-                    solve(1, need, left, xleft, FL, XL);
-                    // s_fl was last read before the primitive barrier of this plane
-                    if (in_block) {
+                        for (int f = 0; f < NFX; ++f) xleft.f[f] = s_prim[pb ^ 1][NV + f][hyl + 1][hx + 1];
+                        solve(1, left, xleft, FL, XL, pl, qL);
+                        // s_fl was last read before the primitive barrier of this plane
 #pragma unroll
-                        for (int v = 0; v < NV; ++v) s_fl[0][v][hy][hx] = FL[v];
+                        for (int v = 0; v < NV; ++v) s_fl[v][hy][hx] = FL[v];
 #pragma unroll
-                        for (int f = 0; f < NFX; ++f) s_fl[0][NV + f][hy][hx] = XL.f[f];
+                        for (int f = 0; f < NFX; ++f) s_fl[NV + f][hy][hx] = XL.f[f];
+                        if constexpr (kFaceP) {
+#pragma unroll
+                            for (int v = 2; v < NV; ++v) s_fp[v - 2][hy][hx] = pl[v];
+                        }
                     }
                     __syncthreads();
-                    if (out_col) {
+                    if (live) {
+                        int const hyr = min(hy + 1, HY - 1);
 #pragma unroll
-                        for (int v = 0; v < NV; ++v) FR[v] = s_fl[0][v][hy + 1][hx];
+                        for (int v = 0; v < NV; ++v) FR[v] = s_fl[v][hyr][hx];
 #pragma unroll
-                        for (int f = 0; f < NFX; ++f) XR.f[f] = s_fl[0][NV + f][hy + 1][hx];
-                        accumulate(1, FL, FR, XL, XR);
+                        for (int f = 0; f < NFX; ++f) XR.f[f] = s_fl[NV + f][hyr][hx];
+                        if constexpr (kFaceP) {
+                            qR[0] = fs[1][1][0];
+#pragma unroll
+                            for (int v = 2; v < NV; ++v) qR[v] = s_fp[v - 2][hyr][hx];
+                        }
+                        accumulate(1, FL, FR, XL, XR, qL, qR);
                     }
                 }
             }
             // geometric pressure source of the march dim (1D spherical: r; 2D spherical: theta)
             if constexpr (GEOM == kSpherical && MD <= 1) {
-                if (out_col) {
+                if (live) {
                     State<ND, T> const pL = cons_to_prim(fs[0][MD], eos);
                     State<ND, T> const pR = cons_to_prim(fs[1][MD], eos);
                     T const dS = T(face_area<ND, GEOM>(G, MD, ci, cj, ck));
@@ -800,7 +792,7 @@ __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM>())) void k_step
         }
 
         // ---- march-dim face h-1/2 and completion of plane h-1
-        if (h >= zs && out_col) {
+        if (h >= zs && live) {
             if constexpr (kPark) {
 #pragma unroll
                 for (int v = 0; v < NV; ++v) fsR_prev[v] = unpark(v);
@@ -836,24 +828,31 @@ __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM>())) void k_step
 #pragma unroll
                 for (int v = 0; v < NV; ++v) un[v] += dtodv_m * ((Fm_prev[v] * dS) - (Fm[v] * dSp));
                 if constexpr (GEOM == kSpherical && MD <= 1) un[1 + MD] += src_prev;
-                T const g = T(gravity(G, pi, MD));
-                un[1 + MD] += dt * g * old_rho_prev;
-                un[ND + 1] += dt * g * old_mom_prev;
-                if (!A.scalars_only) store_cons<ND>(A, G, cell_at<ND>(G, a, bb, hm), un);
-                if constexpr (NFX > 0) {  // godunov_scheme.hpp:288, then passive_scalar_Godunov (:294-301)
-                    int64_t const id = cell_at<ND>(G, a, bb, hm);
+                if (gravity_acts(G, MD)) {
+                    T const g = T(gravity(G, pi, MD));
+                    un[1 + MD] += dt * g * old_rho_prev;
+                    un[ND + 1] += dt * g * old_mom_prev;
+                }
+                if (out_col) {
+                    if (!A.scalars_only) store_cons<ND>(A, G, cell_at<ND>(G, a, bb, hm), un);
+                    if constexpr (NFX > 0) {  // godunov_scheme.hpp:288, then passive_scalar_Godunov (:294-301)
+                        int64_t const id = cell_at<ND>(G, a, bb, hm);
 #pragma unroll
-                    for (int f = 0; f < NFX; ++f) {
-                        T const xn = xpart_prev.f[f] + dtodv_m * ((ffm_prev.f[f] * dS) - (XFm.f[f] * dSp));
-                        T const y = Eos::div(xn, un[0]);
-                        A.fx_new[id + G.plane * f] = y < T(0) ? T(0) : (y > T(1) ? T(1) : y);
+                        for (int f = 0; f < NFX; ++f) {
+                            T const xn = xpart_prev.f[f] + dtodv_m * ((ffm_prev.f[f] * dS) - (XFm.f[f] * dSp));
+                            T const y = Eos::div(xn, un[0]);
+                            A.fx_new[id + G.plane * f] = y < T(0) ? T(0) : (y > T(1) ? T(1) : y);
+                        }
+                    }
+                    // epilogue: CFL rate of the new state and the conserved totals (FP64); a cell the
+                    // pressure fix rewrites gets its rate from k_pressure_fix_fused
+                    if (!pf_prev) r_inv = reduce_combine<kMax>(r_inv, state_rate<ND, GEOM>(G, eos, pi, pj, pk, un));
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) {
+                        if (v < kSumLds) s_sum[v][tid] += (double)un[v] * vol;
+                        else r_sum[v] += (double)un[v] * vol;
                     }
                 }
-                // epilogue: CFL rate of the new state and the conserved totals (FP64); a cell the
-                // pressure fix rewrites gets its rate from k_pressure_fix_fused
-                if (!pf_prev) r_inv = reduce_combine<kMax>(r_inv, state_rate<ND, GEOM>(G, eos, pi, pj, pk, un));
-#pragma unroll
-                for (int v = 0; v < NV; ++v) r_sum[v] += (double)un[v] * vol;
             }
             if constexpr (kPark) {
 #pragma unroll
@@ -904,7 +903,7 @@ __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM>())) void k_step
     r_inv = block_reduce<kMax>(r_inv, s_red, tid, NT);
     r_emin = block_reduce<kMin>(r_emin, s_red, tid, NT);
 #pragma unroll
-    for (int v = 0; v < NV; ++v) r_sum[v] = block_reduce<kSum>(r_sum[v], s_red, tid, NT);
+    for (int v = 0; v < NV; ++v) r_sum[v] = block_reduce<kSum>(v < kSumLds ? s_sum[v < kSumLds ? v : 0][tid] : r_sum[v], s_red, tid, NT);
     static_assert(2 + NV < kPartialStride, "the pressure-fix flag has a slot of its own");
     if (tid == 0 && !A.scalars_only) {
         double* out = A.partials + (int64_t)blockIdx.x * kPartialStride;

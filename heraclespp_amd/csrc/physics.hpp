@@ -80,6 +80,70 @@ __host__ __device__ __forceinline__ double fdiv(double a, double b)
 #endif
 }
 
+// Quotients that share a divisor.  recip(b) is fdiv's reciprocal, recip_near(b, y0) the same from
+// a y0 already within a few ulp of 1 / b (the last of fdiv's two Newton steps squares that error,
+// far below an ulp, so both end at the same double) and quot(a, b, y) the rest of fdiv:
+// bit-identical to fdiv(a, b) on its range.  v_rcp_f64 issues in 16.6 cycles on MI355X where an
+// FP64 fma takes 4.8 (measured), so a reciprocal from scratch costs 7.5 fma and one from a
+// neighbour (1 / (rho kb) from 1 / rho) three; one that depends on the grid or the equation of
+// state alone is read from a table or a kernel argument.
+__host__ __device__ __forceinline__ double recip(double b)
+{
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(HCLPP_IEEE_DIVISION)
+    double y = __builtin_amdgcn_rcp(b);
+    double e = __builtin_fma(-b, y, 1.0);
+    y = __builtin_fma(y, e, y);
+    e = __builtin_fma(-b, y, 1.0);
+    return __builtin_fma(y, e, y);
+#else
+    return 1 / b;
+#endif
+}
+
+__host__ __device__ __forceinline__ double recip_near(double b, double y0)
+{
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(HCLPP_IEEE_DIVISION)
+    double const e = __builtin_fma(-b, y0, 1.0);
+    return __builtin_fma(y0, e, y0);
+#else
+    return 1 / b;
+#endif
+}
+
+__host__ __device__ __forceinline__ double quot(double a, double b, double y)
+{
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(HCLPP_IEEE_DIVISION)
+    double const q = a * y;
+    double const r = __builtin_fma(-b, q, a);
+    return __builtin_amdgcn_div_fixup(__builtin_fma(r, y, q), b, a);
+#else
+    return a / b;
+#endif
+}
+
+// Square root of a squared speed: the sequence hipcc emits for an IEEE square root on gfx950
+// (v_rsq_f64, one coupled Newton step for root and half reciprocal, two remainder corrections)
+// without the two v_ldexp_f64 that scale arguments below 2^-767, so bit-identical to sqrt for
+// zero, infinity, NaN, negative arguments and every argument from 2^-767 on.
+__host__ __device__ __forceinline__ double speed_sqrt(double x)
+{
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(HCLPP_IEEE_DIVISION)
+    double const y = __builtin_amdgcn_rsq(x);
+    double g = x * y;
+    double h = y * 0.5;
+    double const r = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, r, g);
+    h = __builtin_fma(h, r, h);
+    double d = __builtin_fma(-g, g, x);
+    g = __builtin_fma(d, h, g);
+    d = __builtin_fma(-g, g, x);
+    g = __builtin_fma(d, h, g);
+    return __builtin_isfpclass(x, 0x260) ? x : g;  // +-0, +infinity
+#else
+    return sqrt(x);
+#endif
+}
+
 enum Limiter { kConstant = 0, kVanLeer = 1, kMinmod = 2, kVanAlbada = 3 };
 enum Solver { kHLL = 0, kHLLC = 1, kLowMach = 2 };
 enum Geom { kCartesian = 0, kSpherical = 1 };
@@ -108,43 +172,69 @@ struct PerfectGas {
     double gamma;
     double gamma_m1;
     double mmw;
+    // divisors of the temperature round trip and their reciprocals, formed once on the host (make);
+    // the host build divides and leaves them alone
+    double mmw_mp = 0, y_pres = 0;      // mmw mp
+    double mmw_mp_gm1 = 0, y_evol = 0;  // mmw mp (gamma - 1)
+
+    static PerfectGas make(double gamma, double mmw)
+    {
+        PerfectGas g{gamma, gamma - 1, mmw};  // perfect_gas.cpp:13
+        g.mmw_mp = mmw * kMp;
+        g.y_pres = 1 / g.mmw_mp;
+        g.mmw_mp_gm1 = mmw * kMp * g.gamma_m1;
+        g.y_evol = 1 / g.mmw_mp_gm1;
+        return g;
+    }
+#if defined(__HIP_DEVICE_COMPILE__)
+    __device__ __forceinline__ double c_pres() const { return mmw_mp; }
+    __device__ __forceinline__ double c_evol() const { return mmw_mp_gm1; }
+#else
+    __host__ __forceinline__ double c_pres() const { return mmw * kMp; }
+    __host__ __forceinline__ double c_evol() const { return mmw * kMp * gamma_m1; }
+#endif
+    // a / b for a positive grid length b whose reciprocal y a table holds
+    __host__ __device__ static __forceinline__ double quot_grid(double a, double b, double y) { return quot(a, b, y); }
+    __host__ __device__ static __forceinline__ double quot_const(double a, double b, double y) { return quot(a, b, y); }
 
     __host__ __device__ static __forceinline__ double div(double a, double b) { return fdiv(a, b); }
     // IEEE division for the slope limiters, whose operands range over every magnitude (fdiv above)
     __host__ __device__ static __forceinline__ double ratio(double a, double b) { return a / b; }
     // perfect_gas.hpp:69-72
     __host__ __device__ __forceinline__ double temp_from_pres(double rho, double P) const { return fdiv(P * mmw * kMp, rho * kKb); }
-    // perfect_gas.hpp:52-56
-    __host__ __device__ __forceinline__ double evol_from_temp(double rho, double T) const { return fdiv(rho * kKb * T, mmw * kMp * gamma_m1); }
-    // perfect_gas.hpp:46-50
-    __host__ __device__ __forceinline__ double evol_from_pres(double rho, double P) const { return evol_from_temp(rho, temp_from_pres(rho, P)); }
-    // perfect_gas.hpp:74-78
-    __host__ __device__ __forceinline__ double temp_from_evol(double rho, double evol) const
+    // perfect_gas.hpp:52-56 and :46-50: rho kb (its reciprocal yb), then the temperature round trip
+    __host__ __device__ __forceinline__ double evol_from_pres(double rho, double P, double yb) const
     {
-        return fdiv(evol * mmw * kMp * gamma_m1, rho * kKb);
+        double const b = rho * kKb;
+        double const T = quot(P * mmw * kMp, b, yb);
+        return quot_const(b * T, c_evol(), y_evol);
     }
-    // perfect_gas.hpp:64-67
-    __host__ __device__ __forceinline__ double pres_from_temp(double rho, double T) const { return fdiv(rho * kKb * T, mmw * kMp); }
-    // perfect_gas.hpp:58-62
-    __host__ __device__ __forceinline__ double pres_from_evol(double rho, double evol) const
+    __host__ __device__ __forceinline__ double evol_from_pres(double rho, double P) const { return evol_from_pres(rho, P, recip(rho * kKb)); }
+    // reciprocal of rho kb from that of rho
+    __host__ __device__ static __forceinline__ double recip_kb(double rho, double yrho) { return recip_near(rho * kKb, yrho * (1 / kKb)); }
+    // perfect_gas.hpp:74-78, :64-67 and :58-62
+    __host__ __device__ __forceinline__ double pres_from_evol(double rho, double evol, double yb) const
     {
-        return pres_from_temp(rho, temp_from_evol(rho, evol));
+        double const b = rho * kKb;
+        double const T = quot(evol * mmw * kMp * gamma_m1, b, yb);
+        return quot_const(b * T, c_pres(), y_pres);
     }
     // perfect_gas.hpp:80-83
     __host__ __device__ __forceinline__ double sound(double rho, double P) const { return sqrt(fdiv(gamma * P, rho)); }
-    // euler_equations.hpp:61-65, :111-122: pressure of a conservative state
+    __host__ __device__ __forceinline__ double sound(double rho, double P, double y) const { return speed_sqrt(quot(gamma * P, rho, y)); }
+    // euler_equations.hpp:61-65, :111-122: pressure of a conservative state (y: reciprocal of its
+    // density), also returning the internal energy E - |m|^2 / 2 rho it is recovered from
+    template <int ND>
+    __host__ __device__ __forceinline__ double pressure_of_cons(const State<ND, double>& c, double y, double& evol) const
+    {
+        evol = c[ND + 1] - kinetic_cons_with(c, [y](double a, double b) { return quot(a, b, y); });
+        return pres_from_evol(c[0], evol, recip_kb(c[0], y));
+    }
     template <int ND>
     __host__ __device__ __forceinline__ double pressure_of_cons(const State<ND, double>& c) const
     {
-        double const evol = c[ND + 1] - kinetic_cons_with(c, div);
-        return pres_from_evol(c[0], evol);
-    }
-    // the same, also returning the internal energy E - |m|^2 / 2 rho it recovers the pressure from
-    template <int ND>
-    __host__ __device__ __forceinline__ double pressure_of_cons(const State<ND, double>& c, double& evol) const
-    {
-        evol = c[ND + 1] - kinetic_cons_with(c, div);
-        return pres_from_evol(c[0], evol);
+        double evol;
+        return pressure_of_cons(c, recip(c[0]), evol);
     }
     template <int ND>
     __host__ __device__ __forceinline__ double internal_energy_fp64(const State<ND, double>& c) const
@@ -171,6 +261,7 @@ struct PerfectGasMixed {
 #endif
     }
     __host__ __device__ static __forceinline__ float ratio(float a, float b) { return div(a, b); }
+    __host__ __device__ static __forceinline__ float quot_grid(float a, double, double y) { return a * (float)y; }
     __host__ __device__ __forceinline__ float evol_from_pres(float, float P) const { return P * inv_gamma_m1; }
     __host__ __device__ __forceinline__ float sound(float rho, float P) const { return sqrtf(gamma * div(P, rho)); }
     // E - |m|^2 / (2 rho) and (gamma - 1) times it, in FP64
@@ -224,6 +315,7 @@ struct PerfectGasFast {
 #endif
     }
     __host__ __device__ static __forceinline__ double ratio(double a, double b) { return div(a, b); }
+    __host__ __device__ static __forceinline__ double quot_grid(double a, double, double y) { return a * y; }
     __host__ __device__ __forceinline__ double evol_from_pres(double, double P) const { return P * inv_gamma_m1; }
     __host__ __device__ __forceinline__ double sound(double rho, double P) const { return sqrt(gamma * div(P, rho)); }
     template <int ND>
@@ -276,30 +368,72 @@ __host__ __device__ __forceinline__ double internal_energy(const State<ND, doubl
     return c[ND + 1] - kinetic_cons(c);
 }
 
-// euler_equations.hpp:111-122
+// euler_equations.hpp:111-122, also returning the internal energy of the state (in FP64 for
+// every policy), which the pressure recovery forms anyway (internal_energy.cpp:25-40 computes the
+// same value), and with PerfectGas the reciprocal y of the density
 template <int ND, class Eos>
-__host__ __device__ __forceinline__ State<ND, typename Eos::real> cons_to_prim(const State<ND, typename Eos::real>& c, const Eos& eos)
+__host__ __device__ __forceinline__ State<ND, typename Eos::real> cons_to_prim_ey(const State<ND, typename Eos::real>& c, const Eos& eos,
+                                                                                 double& evol, double& y)
 {
     State<ND, typename Eos::real> p;
     p[0] = c[0];
+    if constexpr (std::is_same_v<Eos, PerfectGas>) {
+        y = recip(c[0]);
 #pragma unroll
-    for (int d = 0; d < ND; ++d) p[1 + d] = Eos::div(c[1 + d], c[0]);
-    p[ND + 1] = eos.pressure_of_cons(c);
+        for (int d = 0; d < ND; ++d) p[1 + d] = quot(c[1 + d], c[0], y);
+        p[ND + 1] = eos.pressure_of_cons(c, y, evol);
+    } else {
+        y = 0;
+#pragma unroll
+        for (int d = 0; d < ND; ++d) p[1 + d] = Eos::div(c[1 + d], c[0]);
+        p[ND + 1] = eos.pressure_of_cons(c, evol);
+    }
     return p;
 }
 
-// cons_to_prim that also returns the internal energy of the state (in FP64 for both policies),
-// which the pressure recovery forms anyway (internal_energy.cpp:25-40 computes the same value)
 template <int ND, class Eos>
 __host__ __device__ __forceinline__ State<ND, typename Eos::real> cons_to_prim_e(const State<ND, typename Eos::real>& c, const Eos& eos,
                                                                                 double& evol)
 {
+    double y;
+    return cons_to_prim_ey(c, eos, evol, y);
+}
+
+template <int ND, class Eos>
+__host__ __device__ __forceinline__ State<ND, typename Eos::real> cons_to_prim(const State<ND, typename Eos::real>& c, const Eos& eos)
+{
+    double evol, y;
+    return cons_to_prim_ey(c, eos, evol, y);
+}
+
+// One side of a Riemann problem: primitives, sound speed and, with PerfectGas, the reciprocal yb of
+// rho kb that the side's physical flux needs again.
+template <int ND, class Eos>
+struct FaceSide {
     State<ND, typename Eos::real> p;
-    p[0] = c[0];
+    typename Eos::real s;
+    double yb;
+};
+
+template <int ND, class Eos>
+__host__ __device__ __forceinline__ FaceSide<ND, Eos> face_side(const State<ND, typename Eos::real>& c, const Eos& eos)
+{
+    FaceSide<ND, Eos> f;
+    if constexpr (std::is_same_v<Eos, PerfectGas>) {
+        double const y = recip(c[0]);
+        f.yb = PerfectGas::recip_kb(c[0], y);
+        f.p[0] = c[0];
 #pragma unroll
-    for (int d = 0; d < ND; ++d) p[1 + d] = Eos::div(c[1 + d], c[0]);
-    p[ND + 1] = eos.pressure_of_cons(c, evol);
-    return p;
+        for (int d = 0; d < ND; ++d) f.p[1 + d] = quot(c[1 + d], c[0], y);
+        double const evol = c[ND + 1] - kinetic_cons_with(c, [y](double a, double b) { return quot(a, b, y); });
+        f.p[ND + 1] = eos.pres_from_evol(c[0], evol, f.yb);
+        f.s = eos.sound(c[0], f.p[ND + 1], y);
+    } else {
+        f.p = cons_to_prim(c, eos);
+        f.s = eos.sound(f.p[0], f.p[ND + 1]);
+        f.yb = 0;
+    }
+    return f;
 }
 
 // euler_equations.hpp:124-134
@@ -336,6 +470,18 @@ __host__ __device__ __forceinline__ State<ND, typename Eos::real> flux_of_prim(c
 {
     using T = typename Eos::real;
     return flux_of_prim_e<ND, T>(p, dir, kinetic_prim(p) + eos.evol_from_pres(p[0], p[ND + 1]));
+}
+
+// the same for one side of a Riemann problem
+template <int ND, class Eos>
+__host__ __device__ __forceinline__ State<ND, typename Eos::real> flux_of_side(const State<ND, typename Eos::real>& p, double yb, int dir,
+                                                                              const Eos& eos)
+{
+    using T = typename Eos::real;
+    if constexpr (std::is_same_v<Eos, PerfectGas>)
+        return flux_of_prim_e<ND, T>(p, dir, kinetic_prim(p) + eos.evol_from_pres(p[0], p[ND + 1], yb));
+    else
+        return flux_of_prim(p, dir, eos);
 }
 
 // euler_equations.hpp:93-109: physical flux along `dir` from a conservative state
@@ -414,20 +560,18 @@ __host__ __device__ __forceinline__ T hll_component(T UL, T UR, T FL, T FR, T ws
 
 // riemann_solver.hpp:30-58
 template <int ND, class Eos>
-__host__ __device__ __forceinline__ State<ND, typename Eos::real> riemann_hll(const State<ND, typename Eos::real>& cL,
-                                                                             const State<ND, typename Eos::real>& cR, int dir, const Eos& eos)
+__host__ __device__ __forceinline__ State<ND, typename Eos::real> riemann_hll(const State<ND, typename Eos::real>& cL, const State<ND, typename Eos::real>& cR,
+    const FaceSide<ND, Eos>& L, const FaceSide<ND, Eos>& R, int dir, const Eos& eos)
 {
     using T = typename Eos::real;
-    State<ND, T> const pL = cons_to_prim(cL, eos);
-    State<ND, T> const pR = cons_to_prim(cR, eos);
-    T const sL = eos.sound(pL[0], pL[ND + 1]);
-    T const sR = eos.sound(pR[0], pR[ND + 1]);
+    State<ND, T> const &pL = L.p, &pR = R.p;
+    T const sL = L.s, sR = R.s;
     T const wsL = fmin(pL[1 + dir] - sL, pR[1 + dir] - sR);
     T const wsR = fmax(pL[1 + dir] + sL, pR[1 + dir] + sR);
     T const nL = fmin(wsL, T(0));
     T const pR_ = fmax(wsR, T(0));
-    State<ND, T> const fL = flux_of_prim(pL, dir, eos);
-    State<ND, T> const fR = flux_of_prim(pR, dir, eos);
+    State<ND, T> const fL = flux_of_side(pL, L.yb, dir, eos);
+    State<ND, T> const fR = flux_of_side(pR, R.yb, dir, eos);
     State<ND, T> f;
 #pragma unroll
     for (int v = 0; v < ND + 2; ++v) f[v] = hll_component<Eos>(cL[v], cR[v], fL[v], fR[v], nL, pR_);
@@ -443,14 +587,12 @@ __host__ __device__ __forceinline__ T hllc_component(T F, T U, T Us, T ws)
 
 // riemann_solver.hpp:70-134
 template <int ND, class Eos>
-__host__ __device__ __forceinline__ State<ND, typename Eos::real> riemann_hllc(const State<ND, typename Eos::real>& cL,
-                                                                              const State<ND, typename Eos::real>& cR, int dir, const Eos& eos)
+__host__ __device__ __forceinline__ State<ND, typename Eos::real> riemann_hllc(const State<ND, typename Eos::real>& cL, const State<ND, typename Eos::real>& cR,
+    const FaceSide<ND, Eos>& L, const FaceSide<ND, Eos>& R, int dir, const Eos& eos)
 {
     using T = typename Eos::real;
-    State<ND, T> const pL = cons_to_prim(cL, eos);
-    State<ND, T> const pR = cons_to_prim(cR, eos);
-    T const sL = eos.sound(pL[0], pL[ND + 1]);
-    T const sR = eos.sound(pR[0], pR[ND + 1]);
+    State<ND, T> const &pL = L.p, &pR = R.p;
+    T const sL = L.s, sR = R.s;
     T const uL = pL[1 + dir];
     T const uR = pR[1 + dir];
     T const wsL = fmin(uL - sL, uR - sR);
@@ -465,7 +607,7 @@ __host__ __device__ __forceinline__ State<ND, typename Eos::real> riemann_hllc(c
     State<ND, T> const& ps = left ? pL : pR;
     // the reference evaluates both physical fluxes and keeps the upwind one; only that one is
     // evaluated here (same expressions on the same state, so the same value)
-    State<ND, T> const fs = flux_of_prim(ps, dir, eos);
+    State<ND, T> const fs = flux_of_side(ps, left ? L.yb : R.yb, dir, eos);
     T const un = ps[1 + dir];
     if (wsL * wsR > 0) return fs;
     State<ND, T> f;
@@ -481,14 +623,12 @@ __host__ __device__ __forceinline__ State<ND, typename Eos::real> riemann_hllc(c
 
 // riemann_solver.hpp:146-180 ("Low Mach" splitting solver)
 template <int ND, class Eos>
-__host__ __device__ __forceinline__ State<ND, typename Eos::real> riemann_lowmach(const State<ND, typename Eos::real>& cL,
-                                                                                 const State<ND, typename Eos::real>& cR, int dir, const Eos& eos)
+__host__ __device__ __forceinline__ State<ND, typename Eos::real> riemann_lowmach(const State<ND, typename Eos::real>& cL, const State<ND, typename Eos::real>& cR,
+    const FaceSide<ND, Eos>& L, const FaceSide<ND, Eos>& R, int dir, const Eos& eos)
 {
     using T = typename Eos::real;
-    State<ND, T> const pL = cons_to_prim(cL, eos);
-    State<ND, T> const pR = cons_to_prim(cR, eos);
-    T const sL = eos.sound(pL[0], pL[ND + 1]);
-    T const sR = eos.sound(pR[0], pR[ND + 1]);
+    State<ND, T> const &pL = L.p, &pR = R.p;
+    T const sL = L.s, sR = R.s;
     T const a = T(1.1) * fmax(pL[0] * sL, pR[0] * sR);
     T const ustar = ((pL[1 + dir] + pR[1 + dir]) * T(0.5)) - (Eos::div(T(1), 2 * a) * (pR[ND + 1] - pL[ND + 1]));
     T const Ma = Eos::div(fabs(ustar), fmin(sL, sR));
@@ -504,17 +644,26 @@ __host__ __device__ __forceinline__ State<ND, typename Eos::real> riemann_lowmac
     return f;
 }
 
+// Flux through the face between cL and cR, whose primitives L and R the caller has formed (face_side).
+template <int RS, int ND, class Eos>
+__host__ __device__ __forceinline__ State<ND, typename Eos::real> riemann(const State<ND, typename Eos::real>& cL,
+                                                                         const State<ND, typename Eos::real>& cR, const FaceSide<ND, Eos>& L,
+                                                                         const FaceSide<ND, Eos>& R, int dir, const Eos& eos)
+{
+    if constexpr (RS == kHLL) {
+        return riemann_hll(cL, cR, L, R, dir, eos);
+    } else if constexpr (RS == kHLLC) {
+        return riemann_hllc(cL, cR, L, R, dir, eos);
+    } else {
+        return riemann_lowmach(cL, cR, L, R, dir, eos);
+    }
+}
+
 template <int RS, int ND, class Eos>
 __host__ __device__ __forceinline__ State<ND, typename Eos::real> riemann(const State<ND, typename Eos::real>& cL,
                                                                          const State<ND, typename Eos::real>& cR, int dir, const Eos& eos)
 {
-    if constexpr (RS == kHLL) {
-        return riemann_hll(cL, cR, dir, eos);
-    } else if constexpr (RS == kHLLC) {
-        return riemann_hllc(cL, cR, dir, eos);
-    } else {
-        return riemann_lowmach(cL, cR, dir, eos);
-    }
+    return riemann<RS>(cL, cR, face_side(cL, eos), face_side(cR, eos), dir, eos);
 }
 
 // ---------------------------------------------------------------- spherical sources
