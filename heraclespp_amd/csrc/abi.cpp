@@ -509,19 +509,10 @@ int hclpp_hydro_reconstruction(hclpp_ctx* c, int limiter, const hclpp_range* r, 
     if (limiter < 0 || limiter > 3) return fail(HCLPP_ERR_ARG, "Unknown face reconstruction algorithm");
     int rc = check_range(c, r, 1);
     if (rc) return rc;
-    int const nd = c->cfg.ndim, nfx = c->cfg.nfx;
-    int64_t const pl = c->G.plane;
-    Range3 const R = to_range(r);
-    // hydro_reconstruction.hpp:99-109
-    launch_face_reconstruction(nd, limiter, c->G, R, rho, rho_rec, c->stream);
-    for (int d = 0; d < nd; ++d) launch_face_reconstruction(nd, limiter, c->G, R, u + pl * d, u_rec + pl * 2 * nd * d, c->stream);
-    launch_face_reconstruction(nd, limiter, c->G, R, P, P_rec, c->stream);
-    for (int f = 0; f < nfx; ++f) launch_face_reconstruction(nd, limiter, c->G, R, fx + pl * f, fx_rec + pl * 2 * nd * f, c->stream);
-    // :111-126
-    launch_face_prim_to_cons(nd, c->G, R, c->eos, rho_rec, u_rec, P_rec, rhou_rec, E_rec, c->stream);
-    HCLPP_LAUNCHED("face_reconstruction / conv_prim_to_cons");
-    // :128
-    return hancock_impl(c, r, dt, u_rec, P_rec, rho_rec, rhou_rec, E_rec, fx_rec);
+    launch_muscl_hancock(c->cfg.ndim, c->cfg.geom, limiter, c->G, to_range(r), c->eos, dt, rho, u, P, fx, rho_rec, rhou_rec, E_rec, fx_rec, P_rec,
+                         u_rec, c->cfg.nfx, c->stream);  // hydro_reconstruction.hpp:99-128
+    HCLPP_LAUNCHED("hydro_reconstruction");
+    return HCLPP_OK;
 }
 
 int hclpp_godunov(hclpp_ctx* c, int riemann, const hclpp_range* r, double dt, const double* rho, const double* rhou, const double* E,

@@ -87,6 +87,10 @@ void launch_face_prim_to_cons(int nd, const GridDev& G, const Range3& r, const P
 void launch_hancock(int nd, int geom, const GridDev& G, const Range3& r, const PerfectGas& eos, double dt, const double* u_rec,
                     const double* P_rec, double* rho_rec, double* rhou_rec, double* E_rec, double* fx_rec, const double* fx_rec_old,
                     int nfx, hipStream_t s);
+// face_reconstruction, prim -> cons of the face states and the half step in one kernel
+void launch_muscl_hancock(int nd, int geom, int lim, const GridDev& G, const Range3& r, const PerfectGas& eos, double dt, const double* rho,
+                          const double* u, const double* P, const double* fx, double* rho_rec, double* rhou_rec, double* E_rec, double* fx_rec,
+                          double* P_rec, double* u_rec, int nfx, hipStream_t s);
 void launch_godunov(int nd, int geom, int rs, const GridDev& G, const Range3& r, const PerfectGas& eos, double dt, const double* rho,
                     const double* rhou, const double* E, const double* fx, const double* rho_rec, const double* rhou_rec,
                     const double* E_rec, const double* fx_rec, double* rho_new, double* rhou_new, double* E_new, double* fx_new, int nfx,

@@ -434,7 +434,7 @@ class MUSCLHancockHydroReconstruction(IHydroReconstruction):
     velocity component, P and each passive scalar, the prim -> cons conversion of every face state, then the
     extrapolation step.  When both strategies are the library's own (LimitedLinearReconstruction and
     HancockExtrapolationReconstruction with this operator's EoS), the same sequence runs as one C-ABI call
-    (hclpp_hydro_reconstruction), which launches the same kernels."""
+    (hclpp_hydro_reconstruction), one kernel with the same arithmetic (the same results, bit for bit)."""
 
     def __init__(self, face_reconstruction: IFaceReconstruction, hancock_reconstruction: IExtrapolationReconstruction,
                  eos: PerfectGas, P_rec, u_rec):

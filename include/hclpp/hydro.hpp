@@ -468,7 +468,7 @@ public:
 // component, P and each passive scalar, the prim -> cons conversion of every face state, then the
 // extrapolation step.  When both strategies are the library's own (LimitedLinearReconstruction and
 // HancockExtrapolationReconstruction with this operator's EoS), the same sequence runs as one
-// C-ABI call (hclpp_hydro_reconstruction), which launches the same kernels.
+// C-ABI call (hclpp_hydro_reconstruction): one kernel with the same arithmetic.
 template <class Gravity>
 class MUSCLHancockHydroReconstruction : public IHydroReconstruction<Gravity>
 {
