@@ -13,6 +13,7 @@ namespace hclpp {
 struct Range3 {
     int b[3];
     int e[3];
+    int row = 0, col = 0;  // array extents of x and y when the range is walked in memory order (in_memory_order), else 0
     __host__ __device__ int64_t count() const
     {
         return (int64_t)(e[0] - b[0]) * (int64_t)(e[1] - b[1]) * (int64_t)(e[2] - b[2]);
@@ -20,21 +21,54 @@ struct Range3 {
 };
 
 // Block of 64 x 4 threads over (x, y); grid z walks k.  x is the fastest
-// (contiguous) index, so a wavefront reads 64 consecutive doubles.
+// (contiguous) index, so a wavefront reads 64 consecutive doubles.  A range in
+// memory order (row > 0) walks each k plane's cells from the first to the last
+// of the range instead, ghost columns in between included (and skipped), from a
+// 128-byte boundary on: 256 consecutive doubles per block.
 constexpr int kBX = 64;
 constexpr int kBY = 4;
+constexpr int kLine = 16;  // doubles per 128-byte line
+
+// Cells a memory-order walk spans per k plane, its alignment slack included.
+__host__ __device__ __forceinline__ int64_t row_span(const Range3& r)
+{
+    return (int64_t)(r.e[1] - r.b[1] - 1) * r.row + (r.e[0] - r.b[0]) + (kLine - 1);
+}
 
 inline dim3 range_grid(const Range3& r)
 {
     int const nx = r.e[0] - r.b[0], ny = r.e[1] - r.b[1], nz = r.e[2] - r.b[2];
+    if (r.row > 0) return dim3((unsigned)((row_span(r) + kBX * kBY - 1) / (kBX * kBY)), 1, (unsigned)nz);
     return dim3((unsigned)((nx + kBX - 1) / kBX), (unsigned)((ny + kBY - 1) / kBY), (unsigned)nz);
+}
+
+// The range walked in memory order where that takes no more threads than 64 x 4 blocks do (rows
+// much longer than the range's would mostly be skipped) and a plane's cells count in 31 bits.
+inline Range3 in_memory_order(const GridDev& G, const Range3& r)
+{
+    Range3 q = r;
+    q.row = G.nwg[0];
+    q.col = G.nwg[1];
+    dim3 const f = range_grid(q), b = range_grid(r);
+    if ((int64_t)f.x > (int64_t)b.x * b.y || (int64_t)G.nwg[0] * G.nwg[1] >= (int64_t)1 << 30) q.row = q.col = 0;
+    return q;
 }
 
 __device__ __forceinline__ bool range_cell(const Range3& r, int& i, int& j, int& k)
 {
+    k = r.b[2] + (int)blockIdx.z;
+    if (r.row > 0) {
+        int64_t const plane = (int64_t)r.row * r.col * k;
+        int64_t const first = plane + (int64_t)r.row * r.b[1] + r.b[0];
+        int64_t const t = (first & ~(int64_t)(kLine - 1)) + (int64_t)blockIdx.x * (kBX * kBY) + threadIdx.x + kBX * threadIdx.y;
+        if (t < first) return false;
+        unsigned const in_plane = (unsigned)(t - plane);
+        j = (int)(in_plane / (unsigned)r.row);
+        i = (int)(in_plane - (unsigned)j * (unsigned)r.row);
+        return i >= r.b[0] && i < r.e[0] && j < r.e[1];
+    }
     i = r.b[0] + (int)(blockIdx.x * kBX + threadIdx.x);
     j = r.b[1] + (int)(blockIdx.y * kBY + threadIdx.y);
-    k = r.b[2] + (int)blockIdx.z;
     return i < r.e[0] && j < r.e[1];
 }
 

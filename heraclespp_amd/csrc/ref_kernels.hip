@@ -623,23 +623,26 @@ __global__ __launch_bounds__(256) void k_fill_ghosts(GridDev G, BcSpec bc, Ghost
 
 static inline bool empty(const Range3& r) { return r.count() <= 0; }
 
-void launch_prim_to_cons(int nd, const GridDev& G, const Range3& r, const PerfectGas& eos, const double* rho, const double* u, const double* P,
+void launch_prim_to_cons(int nd, const GridDev& G, const Range3& range, const PerfectGas& eos, const double* rho, const double* u, const double* P,
                          double* rhou, double* E, hipStream_t s)
 {
-    if (empty(r)) return;
+    if (empty(range)) return;
+    Range3 const r = in_memory_order(G, range);
     HCLPP_ND_SWITCH(nd, hipLaunchKernelGGL(k_prim_to_cons<ND>, range_grid(r), dim3(kBX, kBY), 0, s, G, r, eos, rho, u, P, rhou, E));
 }
 
-void launch_cons_to_prim(int nd, const GridDev& G, const Range3& r, const PerfectGas& eos, const double* rho, const double* rhou,
+void launch_cons_to_prim(int nd, const GridDev& G, const Range3& range, const PerfectGas& eos, const double* rho, const double* rhou,
                          const double* E, double* u, double* P, hipStream_t s)
 {
-    if (empty(r)) return;
+    if (empty(range)) return;
+    Range3 const r = in_memory_order(G, range);
     HCLPP_ND_SWITCH(nd, hipLaunchKernelGGL(k_cons_to_prim<ND>, range_grid(r), dim3(kBX, kBY), 0, s, G, r, eos, rho, rhou, E, u, P));
 }
 
-void launch_face_reconstruction(int nd, int lim, const GridDev& G, const Range3& r, const double* var, double* rec, hipStream_t s)
+void launch_face_reconstruction(int nd, int lim, const GridDev& G, const Range3& range, const double* var, double* rec, hipStream_t s)
 {
-    if (empty(r)) return;
+    if (empty(range)) return;
+    Range3 const r = in_memory_order(G, range);
 #define HCLPP_LIM_CASE(L) \
     case L: HCLPP_ND_SWITCH(nd, hipLaunchKernelGGL((k_face_reconstruction<ND, L>), range_grid(r), dim3(kBX, kBY), 0, s, G, r, var, rec)); break;
     switch (lim) {
@@ -651,28 +654,31 @@ void launch_face_reconstruction(int nd, int lim, const GridDev& G, const Range3&
 #undef HCLPP_LIM_CASE
 }
 
-void launch_face_prim_to_cons(int nd, const GridDev& G, const Range3& r, const PerfectGas& eos, const double* rho_rec, const double* u_rec,
+void launch_face_prim_to_cons(int nd, const GridDev& G, const Range3& range, const PerfectGas& eos, const double* rho_rec, const double* u_rec,
                               const double* P_rec, double* rhou_rec, double* E_rec, hipStream_t s)
 {
-    if (empty(r)) return;
+    if (empty(range)) return;
+    Range3 const r = in_memory_order(G, range);
     HCLPP_ND_SWITCH(nd, hipLaunchKernelGGL(k_face_prim_to_cons<ND>, range_grid(r), dim3(kBX, kBY), 0, s, G, r, eos, rho_rec, u_rec, P_rec,
                                            rhou_rec, E_rec));
 }
 
-void launch_hancock(int nd, int geom, const GridDev& G, const Range3& r, const PerfectGas& eos, double dt, const double* u_rec,
+void launch_hancock(int nd, int geom, const GridDev& G, const Range3& range, const PerfectGas& eos, double dt, const double* u_rec,
                     const double* P_rec, double* rho_rec, double* rhou_rec, double* E_rec, double* fx_rec, const double* fx_old, int nfx,
                     hipStream_t s)
 {
-    if (empty(r)) return;
+    if (empty(range)) return;
+    Range3 const r = in_memory_order(G, range);
     HCLPP_GEOM_SWITCH(geom, HCLPP_ND_SWITCH(nd, hipLaunchKernelGGL((k_hancock<ND, GEOM>), range_grid(r), dim3(kBX, kBY), 0, s, G, r, eos, dt,
                                                                    u_rec, P_rec, rho_rec, rhou_rec, E_rec, fx_rec, fx_old, nfx)));
 }
 
-void launch_muscl_hancock(int nd, int geom, int lim, const GridDev& G, const Range3& r, const PerfectGas& eos, double dt, const double* rho,
+void launch_muscl_hancock(int nd, int geom, int lim, const GridDev& G, const Range3& range, const PerfectGas& eos, double dt, const double* rho,
                           const double* u, const double* P, const double* fx, double* rho_rec, double* rhou_rec, double* E_rec, double* fx_rec,
                           double* P_rec, double* u_rec, int nfx, hipStream_t s)
 {
-    if (empty(r)) return;
+    if (empty(range)) return;
+    Range3 const r = in_memory_order(G, range);
 #define HCLPP_LIM_CASE(LV)                                                                                                                  \
     case LV:                                                                                                                                \
         HCLPP_GEOM_SWITCH(geom, HCLPP_ND_SWITCH(nd, hipLaunchKernelGGL((k_muscl_hancock<ND, LV, GEOM>), range_grid(r), dim3(kBX, kBY), 0, s, \
@@ -688,11 +694,12 @@ void launch_muscl_hancock(int nd, int geom, int lim, const GridDev& G, const Ran
 #undef HCLPP_LIM_CASE
 }
 
-void launch_godunov(int nd, int geom, int rs, const GridDev& G, const Range3& r, const PerfectGas& eos, double dt, const double* rho,
+void launch_godunov(int nd, int geom, int rs, const GridDev& G, const Range3& range, const PerfectGas& eos, double dt, const double* rho,
                     const double* rhou, const double* E, const double* fx, const double* rho_rec, const double* rhou_rec, const double* E_rec,
                     const double* fx_rec, double* rho_new, double* rhou_new, double* E_new, double* fx_new, int nfx, hipStream_t s)
 {
-    if (empty(r)) return;
+    if (empty(range)) return;
+    Range3 const r = in_memory_order(G, range);
 #define HCLPP_RS_CASE(RSV)                                                                                                         \
     case RSV:                                                                                                                      \
         HCLPP_GEOM_SWITCH(geom, HCLPP_ND_SWITCH(nd, hipLaunchKernelGGL((k_godunov<ND, GEOM, RSV>), range_grid(r), dim3(kBX, kBY), 0, s, G, r, \
