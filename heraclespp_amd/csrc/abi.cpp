@@ -55,6 +55,11 @@ struct hclpp_ctx {
     MarchPlan march {};  // launch plan of the fused kernel
     int march_occ = 0;    // its resident workgroups per CU
     int64_t fused_nb = 0;
+    // passive scalars in a kernel of their own (scalars_apart): its plan, and the mass fluxes between
+    // the two kernels (ndim planes of the storage type)
+    bool scalars_apart = false;
+    MarchPlan scalar_march {};
+    void* mflux = nullptr;
     double* gtab = nullptr;         // radial gravity table (inside tables; rebuilt for internal-mass gravity)
     double* shells = nullptr;       // internal-mass gravity: per-layer sums of rho dV and dV
     double* adj_prim = nullptr;     // reverse step: primitives (NV planes)
@@ -180,6 +185,16 @@ const DevFlag* clock_gate(const hclpp_ctx* c)
 {
     static_assert(offsetof(hclpp_clock, status) == offsetof(hclpp_clock, done) + sizeof(int), "done, status adjacent");
     return reinterpret_cast<const DevFlag*>(&c->clock->pub.done);
+}
+
+// Resident workgroups per CU of the fused kernel a context runs (without the fast arithmetic).
+int fused_occupancy(const hclpp_ctx* c)
+{
+    hclpp_config const& g = c->cfg;
+    bool const f32 = g.precision == HCLPP_FP32_STORAGE;
+    if (g.nfx == 0) return march_occupancy(g.ndim, g.geom, g.riemann, g.limiter, f32);
+    if (c->scalars_apart) return march_occupancy_mass(g.ndim, g.geom, g.riemann, g.limiter, f32);
+    return march_occupancy_fx(g.ndim, g.geom, g.riemann, g.limiter, f32);
 }
 
 int read_scalar(hclpp_ctx* c, double* out)
@@ -361,6 +376,15 @@ int hclpp_ctx_create(const hclpp_config* cfg, hclpp_ctx** out)
     e = hipMemcpy(c->clock, c->host_clock, sizeof(DevClock), hipMemcpyHostToDevice);
     if (e != hipSuccess) return cleanup(hip_fail(e, "hipMemcpy(clock)"));
 
+    // One scalar is carried by the hydro kernel, several go through a kernel of their own after it,
+    // and so does one where the hydro kernel has no registers for it (3D FP64 Cartesian, once the grid
+    // fills the chip).  Runs of 10 steps on MI355X, carried / apart: one scalar 2D 2048^2 3.08 / 3.82 ms,
+    // 3D spherical 160 x 60 x 60 1.85 / 2.35, FP32 128^3 2.10 / 2.51, FP64 50 x 41 x 37 0.69 / 0.74,
+    // 128^3 4.18 / 4.12, 250^3 26.0 / 23.5; two (a hydro kernel per scalar / apart) 2D 2048^2 5.57 / 4.10,
+    // 250^3 49.7 / 25.5, 160 x 60 x 60 3.33 / 2.49.
+    c->scalars_apart = cfg->nfx >= 2
+                       || (cfg->nfx == 1 && nd == 3 && cfg->geom == HCLPP_GEOM_CARTESIAN && cfg->precision == HCLPP_FP64
+                           && (int64_t)G.n[0] * G.n[1] * G.n[2] >= (int64_t)1 << 21);
     // fused-step scratch
     c->shell = make_ghost_shell(G, nd);
     c->ghost_cap = ghost_blocks(c->shell);
@@ -373,9 +397,15 @@ int hclpp_ctx_create(const hclpp_config* cfg, hclpp_ctx** out)
         e = hipGetDevice(&dev);
         if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
         if (e != hipSuccess) return cleanup(hip_fail(e, "hipDeviceGetAttribute(multiProcessorCount)"));
-        int const occ = march_occupancy(nd, cfg->geom, cfg->riemann, cfg->limiter, cfg->precision == HCLPP_FP32_STORAGE, cfg->nfx >= 1);
+        int const occ = fused_occupancy(c);
         c->march = plan_march(G, nd, occ, ncu);
         c->march_occ = occ;
+        if (c->scalars_apart) {
+            bool const f32 = cfg->precision == HCLPP_FP32_STORAGE;
+            c->scalar_march = plan_march(G, nd, scalar_occupancy(nd, cfg->geom, cfg->limiter, cfg->nfx, f32), ncu);
+            e = hipMalloc(&c->mflux, (f32 ? sizeof(float) : sizeof(double)) * G.plane * nd);
+            if (e != hipSuccess) return cleanup(hip_fail(e, "hipMalloc(mass fluxes)"));
+        }
     }
     c->fused_nb = c->march.nb;
     Range3 all;
@@ -397,6 +427,7 @@ int hclpp_ctx_destroy(hclpp_ctx* c)
     if (c->partials) (void)hipFree(c->partials);
     if (c->ghost_partials) (void)hipFree(c->ghost_partials);
     if (c->fix_partials) (void)hipFree(c->fix_partials);
+    if (c->mflux) (void)hipFree(c->mflux);
     if (c->scalars) (void)hipFree(c->scalars);
     if (c->host_scalars) (void)hipHostFree(c->host_scalars);
     if (c->clock) (void)hipFree(c->clock);
@@ -673,7 +704,7 @@ static int fused_step(hclpp_ctx* c, const S* rho, const S* rhou, const S* E, con
     A.fx = nfx > 0 ? fx : nullptr;
     A.fx_new = nfx > 0 ? fx_new : nullptr;
     A.nfx = nfx;
-    A.scalars_only = 0;
+    A.mflux = static_cast<S*>(c->mflux);
     A.pf = f32 ? 0 : c->pf_on;
     A.eps_pf = c->pf_eps;
     A.partials = c->partials;
@@ -690,18 +721,13 @@ static int fused_step(hclpp_ctx* c, const S* rho, const S* rhou, const S* E, con
     }
     bool const timed = c->prof_count < c->prof_max;
     if (timed) HCLPP_HIP(hipEventRecord(c->prof_events[2 * c->prof_count], c->stream));
-    if (nfx > 0) {
-        // one launch of the one-scalar kernel per passive scalar (the scalars do not couple: each
-        // is upwinded with the same mass flux, godunov_scheme.hpp:263-301); the first also writes
-        // the hydro update and the partials
-        for (int f = 0; f < nfx; ++f) {
-            StepArraysT<S> Af = A;
-            Af.fx = fx + c->G.plane * f;
-            Af.fx_new = fx_new + c->G.plane * f;
-            Af.nfx = 1;
-            Af.scalars_only = f > 0;
-            launch_fused_step_fx(nd, c->cfg.geom, c->cfg.riemann, c->cfg.limiter, c->G, c->march, eos, Af, c->stream);
-        }
+    if (nfx > 0 && c->scalars_apart) {
+        // the scalars are upwinded with the hydro step's mass fluxes (godunov_scheme.hpp:263-301) and
+        // do not act on it: the hydro kernel stores those, and the scalar kernel follows
+        launch_fused_step_mass(nd, c->cfg.geom, c->cfg.riemann, c->cfg.limiter, c->G, c->march, eos, A, c->stream);
+        launch_scalar_march(nd, c->cfg.geom, c->cfg.limiter, c->G, c->scalar_march, eos, A, c->stream);
+    } else if (nfx > 0) {
+        launch_fused_step_fx(nd, c->cfg.geom, c->cfg.riemann, c->cfg.limiter, c->G, c->march, eos, A, c->stream);
     } else {
         bool fast = false;
         if constexpr (!f32) fast = c->fast_on;
@@ -802,7 +828,7 @@ int hclpp_set_fast_arithmetic(hclpp_ctx* c, int on)
     if ((on != 0) == (c->fast_on != 0)) return HCLPP_OK;
     int const nd = c->cfg.ndim;
     int const occ = on ? march_occupancy_fast(nd, c->cfg.geom, c->cfg.riemann, c->cfg.limiter)
-                       : march_occupancy(nd, c->cfg.geom, c->cfg.riemann, c->cfg.limiter, false, false);
+                       : march_occupancy(nd, c->cfg.geom, c->cfg.riemann, c->cfg.limiter, false);
     int const rc = replan_march(c, occ);
     if (rc != HCLPP_OK) return rc;
     c->fast_on = on ? 1 : 0;

@@ -41,10 +41,7 @@ struct StepArraysT {
     const S* __restrict__ fx;  // passive scalars (mass fractions, [f][cell]); unused when nfx = 0
     S* __restrict__ fx_new;
     int nfx;
-    // launches after the first of a step with several passive scalars (one scalar per launch, fx
-    // and fx_new pointing at it): the kernel writes that scalar's update only, not the hydro
-    // update or the workgroup partials the first launch wrote
-    int scalars_only;
+    S* __restrict__ mflux;  // mass flux through the face below each cell, [dim][cell] (kStoreMass kernels)
     // pressure fix (FP64 only): cells whose state at time n has E - e_k < eps_pf e_k are left out
     // of the march kernel's CFL maximum; k_pressure_fix_fused rewrites their energy and rate
     int pf;
@@ -97,8 +94,8 @@ struct MarchPlan {
 // per CU, on ncu CUs (see step_fused.hip for the cost model).
 MarchPlan plan_march(const GridDev& G, int nd, int blocks_per_cu, int ncu);
 // Resident workgroups per CU of the k_step_march instance a configuration selects
-// (FP32 storage or not, with the one-scalar kernel or without scalars).
-int march_occupancy(int nd, int geom, int rs, int lim, bool fp32, bool fx);
+// without scalars (FP32 storage or not).
+int march_occupancy(int nd, int geom, int rs, int lim, bool fp32);
 void launch_fused_step(int nd, int geom, int rs, int lim, const GridDev& G, const MarchPlan& P, const PerfectGas& eos, const StepArrays& A,
                        hipStream_t s);
 void launch_fused_step(int nd, int geom, int rs, int lim, const GridDev& G, const MarchPlan& P, const PerfectGasMixed& eos,
@@ -113,6 +110,18 @@ void launch_fused_step_fx(int nd, int geom, int rs, int lim, const GridDev& G, c
 void launch_fused_step_fx(int nd, int geom, int rs, int lim, const GridDev& G, const MarchPlan& P, const PerfectGasMixed& eos,
                           const StepArraysF& A, hipStream_t s);
 int march_occupancy_fx(int nd, int geom, int rs, int lim, bool fp32);
+// the fused step that stores the mass fluxes A.mflux (step_fused_mass.hip), and after it the passive
+// scalars A.nfx of them (step_scalars.hip), which read the mass fluxes and the new density
+void launch_fused_step_mass(int nd, int geom, int rs, int lim, const GridDev& G, const MarchPlan& P, const PerfectGas& eos, const StepArrays& A,
+                            hipStream_t s);
+void launch_fused_step_mass(int nd, int geom, int rs, int lim, const GridDev& G, const MarchPlan& P, const PerfectGasMixed& eos,
+                            const StepArraysF& A, hipStream_t s);
+int march_occupancy_mass(int nd, int geom, int rs, int lim, bool fp32);
+int scalar_groups(int nfx);  // launches of the scalar kernel for nfx scalars
+void launch_scalar_march(int nd, int geom, int lim, const GridDev& G, const MarchPlan& P, const PerfectGas& eos, const StepArrays& A, hipStream_t s);
+void launch_scalar_march(int nd, int geom, int lim, const GridDev& G, const MarchPlan& P, const PerfectGasMixed& eos, const StepArraysF& A,
+                         hipStream_t s);
+int scalar_occupancy(int nd, int geom, int lim, int nfx, bool fp32);
 // the fused step's pressure fix (pressure_fix_fused.hip): after k_step_march, over the march
 // kernel's workgroups (plan P); fix_partials receives two doubles per workgroup
 void launch_pressure_fix_fused(int nd, int geom, int lim, const GridDev& G, const PerfectGas& eos, const StepArrays& A, const MarchPlan& P,

@@ -389,6 +389,10 @@ constexpr int march_min_waves()
     else return GEOM == kSpherical && NFX > 0 ? 1 : 2;
 }
 
+// NFX of a k_step_march that carries no scalars but stores the mass flux through every face
+// (StepArraysT::mflux), for the scalar kernel that follows it (scalar_march.hpp).
+constexpr int kStoreMass = -1;
+
 // Load the NFX passive scalars (mass fractions, layout [f][cell]) of one cell.
 template <int NFX, class S>
 __device__ __forceinline__ Frac<NFX, S> load_frac(const StepArraysT<S>& A, const GridDev& G, int64_t id)
@@ -399,14 +403,16 @@ __device__ __forceinline__ Frac<NFX, S> load_frac(const StepArraysT<S>& A, const
     return x;
 }
 
-// NFX: passive scalars carried through the step (0, or 1 for the kernels of step_fused_fx.hip).
+// NFX: passive scalars carried through the step (0, or 1 for the kernels of step_fused_fx.hip), or
+// kStoreMass.
 template <class Eos, int ND, int GEOM, int RS, int LIM, int NFX, int HX, int HY, int NT>
 __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM, NFX>())) void k_step_march(GridDev G, Eos eos, StepArraysT<typename Eos::real> A, FusedLayout L)
 {
     using T = typename Eos::real;
     using X = Frac<NFX, T>;
     constexpr int NV = ND + 2;
-    constexpr int NL = NV + NFX;             // values per column in the LDS planes
+    constexpr int NS = NFX > 0 ? NFX : 0;    // scalars carried
+    constexpr int NL = NV + NS;              // values per column in the LDS planes
     constexpr int NP = ND - 1;               // in-plane dims
     constexpr int MD = ND - 1;               // march dim
     constexpr int PX = (ND >= 2) ? HX + 2 : 1;
@@ -434,7 +440,7 @@ __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM, NFX>())) void k
     // slots, so no barrier is involved, and the registers are free across the plane's
     // arithmetic.  3D only: in 2D it gained nothing.
     constexpr bool kPark = ND == 3 && !(NFX > 0 && kFp64State<Eos> && GEOM == kSpherical);
-    constexpr int NPARK = kPark ? 3 * NV + 3 * NFX : 1;
+    constexpr int NPARK = kPark ? 3 * NV + 3 * NS : 1;
     __shared__ T s_park[NPARK][kPark ? NT : 1];
 
     DevClock const* clk = A.clock;
@@ -454,6 +460,12 @@ __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM, NFX>())) void k
     // that a column may not need the compiler kept a second, initialised copy of every result of it:
     // 70 register moves per plane of the 3D kernel, 3 % of its time.)
     int const a = ND >= 2 ? min(mc.a, G.nwg[0] - 1) : 0, bb = ND == 3 ? min(mc.bb, G.nwg[1] - 1) : 0;
+    // kStoreMass: the faces whose fluxes this column stores, below its output cells and, from the
+    // column (row) past the last one, above the last output cell
+    bool const in_x = hx >= 1 && hx <= TX && mc.a < G.ngh[0] + G.n[0];
+    bool const in_y = ND < 3 || (hy >= 1 && hy <= TY && mc.bb < G.ngh[1] + G.n[1]);
+    bool const x_face = NFX == kStoreMass && ND >= 2 && in_y && (in_x || (hx >= 1 && mc.a == G.ngh[0] + G.n[0]));
+    bool const y_face = NFX == kStoreMass && ND == 3 && in_x && (in_y || (hy >= 1 && mc.bb == G.ngh[1] + G.n[1]));
     // Waves of a 3D tile all of whose rows lie beyond the last row that needs a predictor (bb = ngh + n)
     // only keep the barriers.
     static_assert(ND == 1 || NT == HX * HY, "one thread per column of the tile");
@@ -468,7 +480,7 @@ __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM, NFX>())) void k
     // 3D spherical FP64 (256 registers): four of the conserved totals live in LDS (the thread's own
     // slots) instead of in registers across the march, as many as two workgroups per CU leave room
     // for (Sedov 7.0 -> 7.4 Gcell/s)
-    constexpr int kSumLds = kPark && kFp64State<Eos> && GEOM == kSpherical && NFX == 0 ? 4 : 0;
+    constexpr int kSumLds = kPark && kFp64State<Eos> && GEOM == kSpherical && NFX <= 0 ? 4 : 0;
     __shared__ double s_sum[kSumLds > 0 ? kSumLds : 1][kSumLds > 0 ? NT : 1];
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
@@ -730,6 +742,9 @@ __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM, NFX>())) void k
 #pragma unroll
                     for (int f = 0; f < NFX; ++f) xleft.f[f] = lane_shift<HX, true>(xf[1][0].f[f]);
                     solve(0, left, xleft, FL, XL, pl, qL);
+                    if constexpr (NFX == kStoreMass) {
+                        if (x_face) A.mflux[cell_at<ND>(G, a, bb, h)] = FL[0];
+                    }
                     // the right face's flux is the left flux of the column at x + 1
 #pragma unroll
                     for (int v = 0; v < NV; ++v) FR[v] = lane_shift<HX, false>(FL[v]);
@@ -753,6 +768,9 @@ __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM, NFX>())) void k
 #pragma unroll
                         for (int f = 0; f < NFX; ++f) xleft.f[f] = s_prim[pb ^ 1][NV + f][hyl + 1][hx + 1];
                         solve(1, left, xleft, FL, XL, pl, qL);
+                        if constexpr (NFX == kStoreMass) {
+                            if (y_face) A.mflux[cell_at<ND>(G, a, bb, h) + G.plane] = FL[0];
+                        }
                         // s_fl was last read before the primitive barrier of this plane
 #pragma unroll
                         for (int v = 0; v < NV; ++v) s_fl[v][hy][hx] = FL[v];
@@ -798,6 +816,9 @@ __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM, NFX>())) void k
                 for (int v = 0; v < NV; ++v) fsR_prev[v] = unpark(v);
             }
             State<ND, T> const Fm = riemann<RS>(fsR_prev, fs[0][MD], MD, eos);
+            if constexpr (NFX == kStoreMass) {  // the face above the last plane belongs to the next segment, or is the last one
+                if (out_col && (h < ze || h == G.ngh[MD] + G.n[MD])) A.mflux[cell_at<ND>(G, a, bb, h) + G.plane * MD] = Fm[0];
+            }
             X XFm;  // upwinded scalar flux of the face h-1/2
 #pragma unroll
             for (int f = 0; f < NFX; ++f) {
@@ -834,7 +855,7 @@ __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM, NFX>())) void k
                     un[ND + 1] += dt * g * old_mom_prev;
                 }
                 if (out_col) {
-                    if (!A.scalars_only) store_cons<ND>(A, G, cell_at<ND>(G, a, bb, hm), un);
+                    store_cons<ND>(A, G, cell_at<ND>(G, a, bb, hm), un);
                     if constexpr (NFX > 0) {  // godunov_scheme.hpp:288, then passive_scalar_Godunov (:294-301)
                         int64_t const id = cell_at<ND>(G, a, bb, hm);
 #pragma unroll
@@ -905,7 +926,7 @@ __global__ __launch_bounds__(NT, (march_min_waves<Eos, ND, GEOM, NFX>())) void k
 #pragma unroll
     for (int v = 0; v < NV; ++v) r_sum[v] = block_reduce<kSum>(v < kSumLds ? s_sum[v < kSumLds ? v : 0][tid] : r_sum[v], s_red, tid, NT);
     static_assert(2 + NV < kPartialStride, "the pressure-fix flag has a slot of its own");
-    if (tid == 0 && !A.scalars_only) {
+    if (tid == 0) {
         double* out = A.partials + (int64_t)blockIdx.x * kPartialStride;
         out[0] = r_inv;
         out[1] = r_emin;

@@ -298,9 +298,8 @@ MarchPlan plan_march(const GridDev& G, int nd, int blocks_per_cu, int ncu)
     return P;
 }
 
-int march_occupancy(int nd, int geom, int rs, int lim, bool fp32, bool fx)
+int march_occupancy(int nd, int geom, int rs, int lim, bool fp32)
 {
-    if (fx) return march_occupancy_fx(nd, geom, rs, lim, fp32);
     int n = 0;
     if (fp32) march_visit(nd, geom, rs, lim, MarchOccupancy<PerfectGasMixed, 0>{&n});
     else march_visit(nd, geom, rs, lim, MarchOccupancy<PerfectGas, 0>{&n});

@@ -244,9 +244,8 @@ int hclpp_step(hclpp_ctx* ctx, const double* rho, const double* rhou, const doub
  * the main loop body of main.cpp:426-457 with nfx > 0, i.e. each scalar reconstructed with the
  * state (hydro_reconstruction.hpp:99-109), carried through the Hancock half step as a partial
  * density (extrapolation_reconstruction.hpp:87-88, 105-108, 315-337), upwinded with the mass
- * flux and clamped to [0, 1] in the update (godunov_scheme.hpp:122, 263-301).  The fused kernel
- * carries one scalar per launch: nfx > 1 launches it nfx times (the first also writes the
- * hydro update), so the hydro arithmetic is repeated per scalar. */
+ * flux and clamped to [0, 1] in the update (godunov_scheme.hpp:122, 263-301).  One scalar
+ * is carried by the hydro kernel; several follow it in a kernel of their own, four per launch. */
 int hclpp_step_fx(hclpp_ctx* ctx, const double* rho, const double* rhou, const double* E, const double* fx, double* rho_new,
                   double* rhou_new, double* E_new, double* fx_new);
 
