@@ -256,6 +256,11 @@ def _ptr(t) -> ctypes.c_void_p:
     return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
 
 
+class _Handle(ctypes.c_void_p):
+    """An hclpp_ctx pointer that keeps its Context alive: `solver().ctx.handle` as a call's argument
+    would otherwise be destroyed before the call reads it."""
+
+
 class Context:
     """An hclpp_ctx: grid tables, EoS, gravity, boundaries and scheme choice on the device."""
 
@@ -316,7 +321,9 @@ class Context:
     @property
     def handle(self):
         lib().hclpp_set_stream(self._h, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
-        return self._h
+        h = _Handle(self._h.value)
+        h.owner = self
+        return h
 
     # shape checks (the reference asserts equal extents)
     def _chk(self, t, lead=(), name="array", dtype=torch.float64):
