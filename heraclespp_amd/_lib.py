@@ -35,7 +35,7 @@ EXPORTS = [
     "hclpp_conv_prim_to_cons", "hclpp_conv_cons_to_prim", "hclpp_face_reconstruction", "hclpp_hancock_extrapolation",
     "hclpp_face_prim_to_cons",
     "hclpp_hydro_reconstruction", "hclpp_godunov", "hclpp_time_step", "hclpp_min_internal_energy", "hclpp_integrate",
-    "hclpp_fill_ghosts", "hclpp_clock_start", "hclpp_clock_read", "hclpp_step", "hclpp_step_fx",
+    "hclpp_fill_ghosts", "hclpp_clock_start", "hclpp_clock_read", "hclpp_step", "hclpp_step_fx", "hclpp_run_steps", "hclpp_run_steps_f32",
     "hclpp_clock_start_f32", "hclpp_step_f32", "hclpp_step_fx_f32",
     "hclpp_cast_f64_to_f32", "hclpp_cast_f32_to_f64", "hclpp_step_dt", "hclpp_clock_record_dt", "hclpp_step_adjoint",
     "hclpp_steps_dt", "hclpp_steps_adjoint", "hclpp_pressure_fix", "hclpp_internal_mass_gravity", "hclpp_gravity_table",
@@ -140,6 +140,8 @@ def lib() -> ctypes.CDLL:
         "hclpp_temperature": [vp, rp, dp, dp, dp],
         "hclpp_step": [vp, dp, dp, dp, dp, dp, dp],
         "hclpp_step_fx": [vp, dp, dp, dp, dp, dp, dp, dp, dp],
+        "hclpp_run_steps": [vp, ip] + [dp] * 8,
+        "hclpp_run_steps_f32": [vp, ip] + [dp] * 8,
         "hclpp_clock_start_f32": [vp, d, ip, d, d, ip, dp, dp, dp],
         "hclpp_step_f32": [vp, dp, dp, dp, dp, dp, dp],
         "hclpp_step_fx_f32": [vp, dp, dp, dp, dp, dp, dp, dp, dp],

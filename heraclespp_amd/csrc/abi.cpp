@@ -754,6 +754,33 @@ static int fused_step(hclpp_ctx* c, const S* rho, const S* rhou, const S* E, con
     HCLPP_LAUNCHED("clock advance");
     return HCLPP_OK;
 }
+
+// n steps alternating between the states a and b (hclpp_run_steps): step by step, or in one launch on
+// a 1D grid that one workgroup holds, for the plain step (no scalars, pressure fix, fast arithmetic or
+// state-dependent gravity, which have kernels of their own, and no timing of single steps).
+template <class S>
+static int run_steps(hclpp_ctx* c, int n, const StateBuffers<S>& a, S* fx_a, const StateBuffers<S>& b, S* fx_b)
+{
+    if (!c) return fail(HCLPP_ERR_ARG, "null context");
+    if (n < 0) return fail(HCLPP_ERR_ARG, "n < 0");
+    bool const plain = c->cfg.precision == (std::is_same_v<S, float> ? HCLPP_FP32_STORAGE : HCLPP_FP64) && c->cfg.nfx == 0 && !fx_a && !fx_b
+                       && !c->pf_on && !c->fast_on && c->cfg.gravity != HCLPP_GRAV_INTERNAL_MASS && c->prof_count >= c->prof_max;
+    bool const buffers = a.rho && a.rhou && a.E && b.rho && b.rhou && b.E && a.rho != b.rho && a.rhou != b.rhou && a.E != b.E;
+    if (n > 1 && plain && buffers && run_1d_fits(c->cfg.ndim, c->G)) {
+        if constexpr (std::is_same_v<S, float>)
+            launch_run_1d(c->cfg.geom, c->cfg.riemann, c->cfg.limiter, c->G, c->eos32, c->bc, c->clock, n, a, b, c->stream);
+        else
+            launch_run_1d(c->cfg.geom, c->cfg.riemann, c->cfg.limiter, c->G, c->eos, c->bc, c->clock, n, a, b, c->stream);
+        HCLPP_LAUNCHED("1D run");
+        return HCLPP_OK;
+    }
+    for (int k = 0; k < n; ++k) {
+        StateBuffers<S> const &from = k % 2 ? b : a, &to = k % 2 ? a : b;
+        int const rc = fused_step<S>(c, from.rho, from.rhou, from.E, k % 2 ? fx_b : fx_a, to.rho, to.rhou, to.E, k % 2 ? fx_a : fx_b);
+        if (rc) return rc;
+    }
+    return HCLPP_OK;
+}
 }  // extern "C++"
 
 static int clock_reset(hclpp_ctx* c, double t0, int iter0, double t_end, double cfl, int max_iter)
@@ -978,6 +1005,18 @@ int hclpp_step_fx(hclpp_ctx* c, const double* rho, const double* rhou, const dou
                   double* E_new, double* fx_new)
 {
     return fused_step<double>(c, rho, rhou, E, fx, rho_new, rhou_new, E_new, fx_new);
+}
+
+int hclpp_run_steps(hclpp_ctx* c, int n, double* rho_a, double* rhou_a, double* E_a, double* fx_a, double* rho_b, double* rhou_b, double* E_b,
+                    double* fx_b)
+{
+    return run_steps<double>(c, n, {rho_a, rhou_a, E_a}, fx_a, {rho_b, rhou_b, E_b}, fx_b);
+}
+
+int hclpp_run_steps_f32(hclpp_ctx* c, int n, float* rho_a, float* rhou_a, float* E_a, float* fx_a, float* rho_b, float* rhou_b, float* E_b,
+                        float* fx_b)
+{
+    return run_steps<float>(c, n, {rho_a, rhou_a, E_a}, fx_a, {rho_b, rhou_b, E_b}, fx_b);
 }
 
 int hclpp_step_dt(hclpp_ctx* c, double dt, const double* rho, const double* rhou, const double* E, double* rho_new, double* rhou_new,

@@ -53,6 +53,14 @@ struct StepArraysT {
 using StepArrays = StepArraysT<double>;
 using StepArraysF = StepArraysT<float>;
 
+// One of the two states that consecutive steps alternate between.
+template <class S>
+struct StateBuffers {
+    S* rho;
+    S* rhou;
+    S* E;
+};
+
 struct FusedLayout {
     int ntile[2];  // in-plane tile counts
     int seglen;    // planes per workgroup along the march dim
@@ -126,6 +134,13 @@ int scalar_occupancy(int nd, int geom, int lim, int nfx, bool fp32);
 // kernel's workgroups (plan P); fix_partials receives two doubles per workgroup
 void launch_pressure_fix_fused(int nd, int geom, int lim, const GridDev& G, const PerfectGas& eos, const StepArrays& A, const MarchPlan& P,
                                double* fix_partials, hipStream_t s);
+// nsteps steps of a small 1D grid in one launch (run_1d.hip), from state a, alternating with b; whether
+// a grid is one of those
+bool run_1d_fits(int nd, const GridDev& G);
+void launch_run_1d(int geom, int rs, int lim, const GridDev& G, const PerfectGas& eos, const BcSpec& bc, DevClock* clock, int nsteps,
+                   const StateBuffers<double>& a, const StateBuffers<double>& b, hipStream_t s);
+void launch_run_1d(int geom, int rs, int lim, const GridDev& G, const PerfectGasMixed& eos, const BcSpec& bc, DevClock* clock, int nsteps,
+                   const StateBuffers<float>& a, const StateBuffers<float>& b, hipStream_t s);
 GhostShell make_ghost_shell(const GridDev& G, int nd);
 int64_t ghost_blocks(const GhostShell& B);
 void launch_ghosts_rate(int nd, int geom, const GridDev& G, const PerfectGas& eos, const BcSpec& bc, const GhostShell& B, const StepArrays& A,

@@ -4,28 +4,12 @@
 
 #include <algorithm>
 
+#include "clock.hpp"
 #include "march.hpp"
 
 namespace hclpp {
 
 // ------------------------------------------------------------ ghost fill + ghost CFL rates
-__device__ __forceinline__ int ghost_map(int kind, int idx, int ng, int n, int ext, bool& flip)
-{
-    if (idx < ng) {
-        if (kind == kPeriodic) return idx + n;
-        if (kind == kNullGradient) return ng;
-        flip = !flip;
-        return (2 * ng) - 1 - idx;
-    }
-    if (idx >= ng + n) {
-        if (kind == kPeriodic) return idx - n;
-        if (kind == kNullGradient) return ext - ng - 1;
-        flip = !flip;
-        return (2 * (ext - ng)) - 1 - idx;
-    }
-    return idx;
-}
-
 template <class Eos, int ND, int GEOM>
 __global__ __launch_bounds__(256) void k_ghosts_rate(GridDev G, Eos eos, BcSpec bc, GhostShell B, StepArraysT<typename Eos::real> A)
 {
@@ -50,7 +34,7 @@ __global__ __launch_bounds__(256) void k_ghosts_rate(GridDev G, Eos eos, BcSpec 
 #pragma unroll
         for (int d = 0; d < ND; ++d) {
             int const side = idx[d] < G.ngh[d] ? 0 : 1;
-            src[d] = ghost_map(bc.kind[2 * d + side], idx[d], G.ngh[d], G.n[d], G.nwg[d], flip[d]);
+            src[d] = face_map(bc.kind[2 * d + side], idx[d], G.ngh[d], G.n[d], G.nwg[d], flip[d]);
         }
         int64_t const dst = flat(G, i, j, k);
         int64_t const s = flat(G, src[0], src[1], src[2]);
@@ -103,44 +87,6 @@ __global__ __launch_bounds__(256) void k_cast(const In* __restrict__ in, Out* __
 }
 
 // ------------------------------------------------------------ clock
-// main.cpp:355-385 (dt, output clipping, t_end clip, max_iter) and :397-425 (internal energy check)
-__device__ __forceinline__ void schedule_next(DevClock* c, double inv)
-{
-    double dt = c->pub.cfl * (1 / inv);
-    int pending = 0, output = 0;
-    if (c->iter_output_frequency > 0) {  // :362-368 (iter_ini = 0)
-        int const next_output = (c->pub.iter_output_id + 1) * c->iter_output_frequency;
-        if ((c->pub.iter + 1) >= next_output) {
-            output = 1;
-            c->pub.iter_output_id += 1;
-        }
-    }
-    if (c->time_output_frequency > 0) {  // :369-375
-        double const next_output = c->time_first_output + ((c->pub.time_output_id + 1) * c->time_output_frequency);
-        if ((c->pub.t + dt) >= next_output) {
-            dt = next_output - c->pub.t;
-            if (dt <= 0) {
-                c->pub.status = HCLPP_ERR_NEGATIVE_DT;
-                return;
-            }
-            output = 1;
-            c->pub.time_output_id += 1;
-        }
-    }
-    if ((c->pub.t + dt) >= c->pub.t_end) {
-        dt = c->pub.t_end - c->pub.t;
-        output = 1;
-        pending = 1;
-    }
-    if ((c->pub.iter + 1) >= c->pub.max_iter) {
-        output = 1;
-        pending = 1;
-    }
-    c->pub.dt = dt;
-    c->pending_exit = pending;
-    c->pending_output = output;
-}
-
 __global__ __launch_bounds__(64) void k_clock_start(DevClock* c, const double* inv)
 {
     if (threadIdx.x == 0) schedule_next(c, inv[0]);
@@ -224,28 +170,7 @@ __global__ __launch_bounds__(1024) void k_clock_advance(DevClock* c, const doubl
 #pragma unroll
         for (int v = 0; v < NV; ++v) s[v] += lds[w][2 + v];
     }
-    c->pub.min_eint = emin;
-    if (isnan(emin) || emin < 0) {
-        c->pub.status = 3;  // HCLPP_ERR_STATE: the step is discarded
-        return;
-    }
-    if (c->dt_log && c->pub.iter < c->dt_log_cap) c->dt_log[c->pub.iter] = c->pub.dt;
-    c->pub.t += c->pub.dt;
-    c->pub.iter += 1;
-    c->pub.mass = s[0];
-    for (int d = 0; d < 3; ++d) c->pub.momentum[d] = d < NV - 2 ? s[1 + d] : 0.;
-    c->pub.energy = s[NV - 1];
-    c->pub.output_due = c->pending_output;
-    if (c->pending_exit) {
-        c->pub.done = 1;
-        c->pub.exiting = 1;
-        return;
-    }
-    if (c->pending_output) {  // pause: the caller writes the output, then starts the clock again
-        c->pub.done = 1;
-        return;
-    }
-    schedule_next(c, inv);
+    clock_finish<NV>(c, inv, emin, s);
 }
 
 // ------------------------------------------------------------ launchers

@@ -224,9 +224,8 @@ class HydroSolver:
             bufs = self._bufs()
             launched = 0
             while True:
-                for _ in range(check_every):
-                    self._launch_step(bufs[(cur0 + launched) % 2], bufs[(cur0 + launched + 1) % 2])
-                    launched += 1
+                self._launch_steps(bufs[(cur0 + launched) % 2], bufs[(cur0 + launched + 1) % 2], check_every)
+                launched += check_every
                 clk = self.clock()
                 if clk.done or clk.status:
                     break
@@ -299,6 +298,12 @@ class HydroSolver:
             step = lib().hclpp_step_f32 if fp32 else lib().hclpp_step
             check(step(self.ctx.handle, _ptr(a[0]), _ptr(a[1]), _ptr(a[2]), _ptr(b[0]), _ptr(b[1]), _ptr(b[2])))
 
+    def _launch_steps(self, a, b, n):
+        """n steps from a, alternating with b (one call: no host work per step)."""
+        run = lib().hclpp_run_steps_f32 if self.precision == "fp32" else lib().hclpp_run_steps
+        fx = [_ptr(s[3]) if self.nfx else ctypes.c_void_p(0) for s in (a, b)]
+        check(run(self.ctx.handle, n, _ptr(a[0]), _ptr(a[1]), _ptr(a[2]), fx[0], _ptr(b[0]), _ptr(b[1]), _ptr(b[2]), fx[1]))
+
     def _sync_back(self):
         if self.precision == "fp32":
             for src, dst in zip(self._cons32[self._cur], self._cons[self._cur]):
@@ -317,9 +322,8 @@ class HydroSolver:
             batch = check_every
             if max_iter - it0 - launched > 0:
                 batch = min(batch, max_iter - it0 - launched)
-            for _ in range(batch):
-                self._launch_step(bufs[(cur0 + launched) % 2], bufs[(cur0 + launched + 1) % 2])
-                launched += 1
+            self._launch_steps(bufs[(cur0 + launched) % 2], bufs[(cur0 + launched + 1) % 2], batch)
+            launched += batch
             clk = self.clock()
             if clk.done or clk.status:
                 break

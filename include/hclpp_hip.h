@@ -262,6 +262,16 @@ int hclpp_step_f32(hclpp_ctx* ctx, const float* rho, const float* rhou, const fl
 /* hclpp_step_fx with FP32 storage (the scalar is stored and computed in FP32). */
 int hclpp_step_fx_f32(hclpp_ctx* ctx, const float* rho, const float* rhou, const float* E, const float* fx, float* rho_new,
                       float* rhou_new, float* E_new, float* fx_new);
+
+/* n steps of hclpp_step (hclpp_step_fx when fx_a and fx_b are given), alternating between two states:
+ * the first reads a and writes b, the next reads b and writes a, ... ; after k steps have run (the
+ * clock may stop earlier than n) the state is in a when k is even, in b when it is odd, and the other
+ * holds no defined state.  One call instead of n; a 1D grid small enough for one workgroup runs them
+ * in one launch.  Results as n calls, except that the clock's totals may be summed in another order. */
+int hclpp_run_steps(hclpp_ctx* ctx, int n, double* rho_a, double* rhou_a, double* E_a, double* fx_a, double* rho_b, double* rhou_b,
+                    double* E_b, double* fx_b);
+int hclpp_run_steps_f32(hclpp_ctx* ctx, int n, float* rho_a, float* rhou_a, float* E_a, float* fx_a, float* rho_b, float* rhou_b,
+                        float* E_b, float* fx_b);
 /* element-wise conversions between FP64 and FP32 device arrays of n values */
 int hclpp_cast_f64_to_f32(hclpp_ctx* ctx, const double* in, float* out, long long n);
 int hclpp_cast_f32_to_f64(hclpp_ctx* ctx, const float* in, double* out, long long n);
