@@ -60,6 +60,7 @@ __device__ __forceinline__ void clock_finish(DevClock* c, double inv, double emi
     c->pub.t += c->pub.dt;
     c->pub.iter += 1;
     c->pub.mass = s[0];
+#pragma unroll
     for (int d = 0; d < 3; ++d) c->pub.momentum[d] = d < NV - 2 ? s[1 + d] : 0.;
     c->pub.energy = s[NV - 1];
     c->pub.output_due = c->pending_output;

@@ -114,7 +114,8 @@ __global__ __launch_bounds__(1024) void k_clock_advance(DevClock* c, const doubl
                                                         const double* __restrict__ fix_partials, int64_t nfix)
 {
     __shared__ double lds[16][NV + 2];  // per-wave results of every reduced value: one LDS round
-    if (c->pub.done || c->pub.status) return;
+    DevClock k = *c;  // read ahead of the reductions, not field by field after them
+    if (k.pub.done || k.pub.status) return;
     double inv = reduce_identity<kMax>(), emin = reduce_identity<kMin>();
     double s[NV];
 #pragma unroll
@@ -132,11 +133,12 @@ __global__ __launch_bounds__(1024) void k_clock_advance(DevClock* c, const doubl
         }
 #pragma unroll
         for (int r = 0; r < kR; ++r) {
-            if (t0 + r * 1024 >= nblocks) break;
-            inv = reduce_combine<kMax>(inv, row[r][0]);
-            emin = reduce_combine<kMin>(emin, row[r][1]);
+            if (t0 + r * 1024 < nblocks) {  // (a break would leave the rows in scratch memory)
+                inv = reduce_combine<kMax>(inv, row[r][0]);
+                emin = reduce_combine<kMin>(emin, row[r][1]);
 #pragma unroll
-            for (int v = 0; v < NV; ++v) s[v] += row[r][2 + v];
+                for (int v = 0; v < NV; ++v) s[v] += row[r][2 + v];
+            }
         }
     }
     for (int64_t t = threadIdx.x; t < nghost; t += 1024) inv = reduce_combine<kMax>(inv, ghost_partials[t]);
@@ -145,8 +147,7 @@ __global__ __launch_bounds__(1024) void k_clock_advance(DevClock* c, const doubl
         inv = reduce_combine<kMax>(inv, fix_partials[2 * t]);
         s[NV - 1] += fix_partials[2 * t + 1];
     }
-    // all NV + 2 values reduced together: wave shuffles, one barrier, then thread 0 folds the
-    // 16 wave results in wave order (a fixed order: the totals are deterministic)
+    // all NV + 2 values reduced together: wave shuffles, one barrier
     inv = wave_reduce<kMax>(inv);
     emin = wave_reduce<kMin>(emin);
 #pragma unroll
@@ -159,18 +160,23 @@ __global__ __launch_bounds__(1024) void k_clock_advance(DevClock* c, const doubl
         for (int v = 0; v < NV; ++v) lds[wave][2 + v] = s[v];
     }
     __syncthreads();
-    if (threadIdx.x != 0) return;
-    inv = reduce_identity<kMax>();
-    emin = reduce_identity<kMin>();
+    // the 16 wave results by lanes of the first wave (a fixed order: the totals are deterministic); one
+    // thread reading all 16 (NV + 2) of them spilled 96 registers
+    if (wave != 0) return;
+    inv = lds[lane & 15][0];
+    emin = lds[lane & 15][1];
 #pragma unroll
-    for (int v = 0; v < NV; ++v) s[v] = 0;
-    for (int w = 0; w < 16; ++w) {
-        inv = reduce_combine<kMax>(inv, lds[w][0]);
-        emin = reduce_combine<kMin>(emin, lds[w][1]);
+    for (int v = 0; v < NV; ++v) s[v] = lds[lane & 15][2 + v];
 #pragma unroll
-        for (int v = 0; v < NV; ++v) s[v] += lds[w][2 + v];
+    for (int o = 8; o > 0; o >>= 1) {
+        inv = reduce_combine<kMax>(inv, __shfl_xor(inv, o, 64));
+        emin = reduce_combine<kMin>(emin, __shfl_xor(emin, o, 64));
+#pragma unroll
+        for (int v = 0; v < NV; ++v) s[v] += __shfl_xor(s[v], o, 64);
     }
-    clock_finish<NV>(c, inv, emin, s);
+    if (lane != 0) return;
+    clock_finish<NV>(&k, inv, emin, s);
+    *c = k;
 }
 
 // ------------------------------------------------------------ launchers
