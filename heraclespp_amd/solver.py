@@ -131,17 +131,15 @@ class HydroSolver:
     def init_from_prim(self, rho, u, P, fx=None, t0: float = 0.0, iter0: int = 0):
         g = self.grid
         nd = g.ndim
-        rho_d = _dev(rho, g.shape3)
-        self.u.copy_(_dev(u, (nd,) + g.shape3))
-        self.P.copy_(_dev(P, g.shape3))
+        rho_d, u_d, P_d = _dev(rho, g.shape3), _dev(u, (nd,) + g.shape3), _dev(P, g.shape3)
         self._cur = 0
         r, m, E = self._cons[0]
         r.copy_(rho_d)
         if self.nfx:
             self.fx.copy_(_dev(fx, (self.nfx,) + g.shape3))
         c = self.ctx
-        check(lib().hclpp_conv_prim_to_cons(c.handle, ctypes.byref(self._r(0)), c._chk(r), c._chk(self.u, (nd,)),
-                                            c._chk(self.P), c._chk(m, (nd,)), c._chk(E)))
+        check(lib().hclpp_conv_prim_to_cons(c.handle, ctypes.byref(self._r(0)), c._chk(r), c._chk(u_d, (nd,)),
+                                            c._chk(P_d), c._chk(m, (nd,)), c._chk(E)))
         check(lib().hclpp_fill_ghosts(c.handle, c._chk(r), c._chk(m, (nd,)), c._chk(E),
                                       c._fx(self.fx, (self.nfx,), "fx")))
         self._refresh_gravity()  # main.cpp:309
