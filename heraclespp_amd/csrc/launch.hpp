@@ -42,15 +42,16 @@ inline dim3 range_grid(const Range3& r)
     return dim3((unsigned)((nx + kBX - 1) / kBX), (unsigned)((ny + kBY - 1) / kBY), (unsigned)nz);
 }
 
-// The range walked in memory order where that takes no more threads than 64 x 4 blocks do (rows
-// much longer than the range's would mostly be skipped) and a plane's cells count in 31 bits.
+// The range walked in memory order where that takes at most an eighth more threads than 64 x 4 blocks
+// do (rows much longer than the range's would mostly be skipped) and a plane's cells count in 31 bits.
+// The aligned lines are worth that: prim -> cons of 512^3, whose rows fill their blocks, 3.03 -> 1.97 ms.
 inline Range3 in_memory_order(const GridDev& G, const Range3& r)
 {
     Range3 q = r;
     q.row = G.nwg[0];
     q.col = G.nwg[1];
     dim3 const f = range_grid(q), b = range_grid(r);
-    if ((int64_t)f.x > (int64_t)b.x * b.y || (int64_t)G.nwg[0] * G.nwg[1] >= (int64_t)1 << 30) q.row = q.col = 0;
+    if ((int64_t)f.x * 8 > (int64_t)b.x * b.y * 9 || (int64_t)G.nwg[0] * G.nwg[1] >= (int64_t)1 << 30) q.row = q.col = 0;
     return q;
 }
 
