@@ -159,7 +159,7 @@ __global__ __launch_bounds__(256) void k_adj_fold(const double* __restrict__ par
 }
 
 struct AdjRanges {
-    Range3 ring2, ring1, interior, flux;  // flux: the union of the face ranges (interior + 1 cell on the high side of every dim)
+    Range3 prim, ring2, ring1, interior, flux;  // flux: the union of the face ranges (interior + 1 cell on the high side of every dim)
 };
 
 AdjRanges adj_ranges(const GridDev& G, int nd)
@@ -176,6 +176,11 @@ AdjRanges adj_ranges(const GridDev& G, int nd)
     }
     R.flux = R.interior;
     for (int d = 0; d < nd; ++d) R.flux.e[d] += 1;
+    // the passes that treat every cell alike walk memory in order; the gather takes blocks, of which the
+    // inner ones skip the search for ghost copies
+    R.prim = in_memory_order(G, R.ring2);
+    R.ring1 = in_memory_order(G, R.ring1);
+    R.flux = in_memory_order(G, R.flux);
     return R;
 }
 
@@ -235,7 +240,7 @@ int64_t launch_step_adjoint(int nd, int geom, int rs, int lim, const GridDev& G,
     Range3 const& rg = R.ring2;
     int64_t off = 0;
     HCLPP_ADJ_ND_SWITCH(nd, HCLPP_ADJ_GEOM_SWITCH(geom, {
-        if (!prims_ready) hipLaunchKernelGGL(k_adj_prim<ND>, range_grid(R.ring2), blk, 0, s, G, R.ring2, eos, A);
+        if (!prims_ready) hipLaunchKernelGGL(k_adj_prim<ND>, range_grid(R.prim), blk, 0, s, G, R.prim, eos, A);
         HCLPP_ADJ_LIM_SWITCH(lim, hipLaunchKernelGGL((k_adj_faces<ND, LIM, GEOM>), range_grid(R.ring1), blk, 0, s, G, R.ring1, eos, A,
                                                      partials, pending, dgamma));
         (launch_flux<ND, GEOM>)(rs, G, R, eos, A, partials, off, s);

@@ -107,6 +107,23 @@ __host__ __device__ __forceinline__ int64_t shifted(const GridDev& G, const int*
     return flat(G, q[0], q[1], q[2]);
 }
 
+// Distances of cell i's center to its neighbours' along d, with their reciprocals: from the grid's
+// table on the device (a division by a tabled reciprocal is three instructions, one without eight),
+// formed on the host, whose quot divides.
+struct Centers {
+    double hm, ym, hp, yp;
+};
+__host__ __device__ __forceinline__ Centers centers(const GridDev& G, int d, int i)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    double const* h = G.hc[d] + 2 * (i - 1);
+    return {h[0], h[1], h[2], h[3]};
+#else
+    double const dl = G.dx[d][i], hm = (G.dx[d][i - 1] + dl) / 2, hp = (dl + G.dx[d][i + 1]) / 2;
+    return {hm, 1 / hm, hp, 1 / hp};
+#endif
+}
+
 // Face primitives of cell c (limited_linear_reconstruction.hpp:46-64), same expressions as the forward.
 template <int ND, int LIM>
 __host__ __device__ __forceinline__ void face_prims(const GridDev& G, const double* prim, const int* c, const S<ND>& p, S<ND> (&pf)[2][ND])
@@ -117,11 +134,10 @@ __host__ __device__ __forceinline__ void face_prims(const GridDev& G, const doub
         S<ND> const pm = load_planes<ND>(prim, shifted(G, c, d, -1), pl, 0);
         S<ND> const pp = load_planes<ND>(prim, shifted(G, c, d, +1), pl, 0);
         double const dl = G.dx[d][c[d]];
-        double const dl_m = G.dx[d][c[d] - 1];
-        double const dl_p = G.dx[d][c[d] + 1];
+        Centers const h = centers(G, d, c[d]);
 #pragma unroll
         for (int v = 0; v < ND + 2; ++v) {
-            double const slope = limited_slope_t<LIM>(fdiv(pp[v] - p[v], (dl + dl_p) / 2), fdiv(p[v] - pm[v], (dl_m + dl) / 2));
+            double const slope = limited_slope_t<LIM>(quot(pp[v] - p[v], h.hp, h.yp), quot(p[v] - pm[v], h.hm, h.ym));
             pf[0][d][v] = p[v] - ((dl / 2) * slope);
             pf[1][d][v] = p[v] + ((dl / 2) * slope);
         }
@@ -342,18 +358,16 @@ __host__ __device__ __forceinline__ void slope_adjoint(const GridDev& G, const d
     S<ND> const pm = load_planes<ND>(prim, shifted(G, c, d, -1), pl, 0);
     S<ND> const pp = load_planes<ND>(prim, shifted(G, c, d, +1), pl, 0);
     double const dl = G.dx[d][c[d]];
-    double const hp = (dl + G.dx[d][c[d] + 1]) / 2;
-    double const hm = (G.dx[d][c[d] - 1] + dl) / 2;
-    double const ihp = fdiv(1, hp), ihm = fdiv(1, hm);
+    Centers const h = centers(G, d, c[d]);
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
         double gR, gL;
         // the forward's slope arguments (they decide the limiter branch): its own divisions
-        limiter_grad<LIM>(fdiv(pp[v] - p[v], hp), fdiv(p[v] - pm[v], hm), gR, gL);
+        limiter_grad<LIM>(quot(pp[v] - p[v], h.hp, h.yp), quot(p[v] - pm[v], h.hm, h.ym), gR, gL);
         double const ls = (dl / 2) * (l1[v] - l0[v]);
         own[v] = l0[v] + l1[v];
-        ra[v] = ls * gR * ihp;
-        rb[v] = ls * gL * ihm;
+        ra[v] = ls * gR * h.yp;
+        rb[v] = ls * gL * h.ym;
     }
 }
 
