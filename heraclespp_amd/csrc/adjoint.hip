@@ -7,7 +7,10 @@
 // In a run of reverse steps, each step's gather pass also forms the primitives the next one
 // needs, so the primitive pass runs once per run, and each step's faces pass folds the
 // previous step's dL/dgamma partials, so the fold runs on its own once per run.
+#include <algorithm>
+
 #include "adjoint_step.hpp"
+#include "fused.hpp"
 #include "reduce.hpp"
 
 namespace hclpp {
@@ -121,24 +124,20 @@ __device__ __forceinline__ bool in_range(const Range3& r, int i, int j, int k)
     return i >= r.b[0] && i < r.e[0] && j >= r.b[1] && j < r.e[1] && k >= r.b[2] && k < r.e[2];
 }
 
-// Gather pass over `rg` (the cells within 2 of the interior): interior cells run the gather;
-// with `nx`, every cell also stores the next state's primitives for the next reverse step (the
-// gather reads no primitive, so the buffer is free).
-template <int ND, int LIM>
+// Gather pass over `rg` (the cells within 2 of the interior): interior cells run the gather, with
+// COPIES the part through the ghosts filled from them too; with `nx`, every cell also stores the next
+// state's primitives for the next reverse step (the gather reads no primitive, so the buffer is free).
+template <int ND, bool COPIES>
 __global__ __launch_bounds__(256) void k_adj_gather(GridDev G, Range3 rg, Range3 interior, PerfectGas eos, BcSpec bc, AdjArrays A, NextState nx,
                                                     double* __restrict__ partials)
 {
-    // a workgroup whose cells all lie where no ghost copies from (adj::no_ghost_copies) takes the
-    // gather without the preimage search; the test is uniform over the workgroup
-    int const i0 = rg.b[0] + (int)blockIdx.x * kBX, j0 = rg.b[1] + (int)blockIdx.y * kBY;
-    bool deep = adj::no_ghost_copies(G, 0, i0, i0 + kBX);
-    if (ND >= 2) deep = deep && adj::no_ghost_copies(G, 1, j0, j0 + kBY);
-    if (ND == 3) deep = deep && adj::no_ghost_copies(G, 2, rg.b[2] + (int)blockIdx.z, rg.b[2] + (int)blockIdx.z + 1);
     int i, j, k;
     double lg = 0;
     if (range_cell(rg, i, j, k)) {
-        if (deep) lg = adj::cell_gather<ND, LIM, true>(G, eos, bc, A, i, j, k);
-        else if (in_range(interior, i, j, k)) lg = adj::cell_gather<ND, LIM>(G, eos, bc, A, i, j, k);
+        if (in_range(interior, i, j, k)) {
+            if constexpr (COPIES) lg = adj::cell_gather<ND, kConstant>(G, eos, bc, A, i, j, k);  // the same for every limiter
+            else lg = adj::gather_self<ND>(G, eos, A, i, j, k);
+        }
         if (nx.rho) {
             AdjArrays B = A;
             B.rho = nx.rho;
@@ -146,6 +145,27 @@ __global__ __launch_bounds__(256) void k_adj_gather(GridDev G, Range3 rg, Range3
             B.E = nx.E;
             adj::cell_prim<ND>(G, eos, B, i, j, k);
         }
+    }
+    put_partial(lg, partials);
+}
+
+// The gather's part through ghost cells, over the interior cells ghosts are filled from (the shell of
+// adj_shell), after k_adj_gather without COPIES.  The search for the ghosts and the neighbour tests of
+// cells outside the interior cost a wave as much for one such cell as for 64, and in memory order every
+// wave of a 96-wide row holds some: 96^3 (walls and periodic sides) 195 us as one pass, 83 + 45 apart.
+template <int ND>
+__global__ __launch_bounds__(256) void k_adj_copies(GridDev G, GhostShell B, PerfectGas eos, BcSpec bc, AdjArrays A, double* __restrict__ partials)
+{
+    int64_t const t = (int64_t)blockIdx.x * kT + threadIdx.x + kBX * threadIdx.y;
+    double lg = 0;
+    if (t < B.start[B.nbox]) {
+        int b = 0;
+        while (t >= B.start[b + 1]) ++b;
+        int64_t loc = t - B.start[b];
+        int const nx = B.hi[b][0] - B.lo[b][0], ny = B.hi[b][1] - B.lo[b][1];
+        int const i = B.lo[b][0] + (int)(loc % nx);
+        loc /= nx;
+        lg = adj::gather_copies<ND>(G, eos, bc, A, i, B.lo[b][1] + (int)(loc % ny), B.lo[b][2] + (int)(loc / ny));
     }
     put_partial(lg, partials);
 }
@@ -159,7 +179,7 @@ __global__ __launch_bounds__(256) void k_adj_fold(const double* __restrict__ par
 }
 
 struct AdjRanges {
-    Range3 prim, ring2, ring1, interior, flux;  // flux: the union of the face ranges (interior + 1 cell on the high side of every dim)
+    Range3 ring2, ring1, interior, flux;  // flux: the union of the face ranges (interior + 1 cell on the high side of every dim)
 };
 
 AdjRanges adj_ranges(const GridDev& G, int nd)
@@ -176,13 +196,49 @@ AdjRanges adj_ranges(const GridDev& G, int nd)
     }
     R.flux = R.interior;
     for (int d = 0; d < nd; ++d) R.flux.e[d] += 1;
-    // the passes that treat every cell alike walk memory in order; the gather takes blocks, of which the
-    // inner ones skip the search for ghost copies
-    R.prim = in_memory_order(G, R.ring2);
+    R.ring2 = in_memory_order(G, R.ring2);
     R.ring1 = in_memory_order(G, R.ring1);
     R.flux = in_memory_order(G, R.flux);
     return R;
 }
+
+// 3D grids whose gather leaves the ghost part to k_adj_copies.  Gradients of 8 steps, in one pass /
+// apart: 40^3 1.69 / 1.81 ms, 56^3 2.30 / 2.26, 96^3 6.17 / 5.99; in 2D, where a boundary cell has a
+// ghost or two, one pass is the faster at any size (1024^2 3.53 / 3.54).
+constexpr int64_t kSplitGather = (int64_t)1 << 17;
+
+// The interior cells that ghosts may be filled from (adj::ghost_copies along some dim), as disjoint boxes.
+GhostShell adj_shell(const GridDev& G, int nd)
+{
+    GhostShell B{};
+    int64_t total = 0;
+    auto low_end = [&](int d) { return std::min(2 * G.ngh[d], G.ngh[d] + G.n[d]); };
+    for (int d = 0; d < nd; ++d)
+        for (int side = 0; side < 2; ++side) {
+            int const b = B.nbox++;
+            int64_t cells = 1;
+            for (int e = 0; e < 3; ++e) {
+                int lo = G.ngh[e], hi = G.ngh[e] + G.n[e];
+                if (e < d) {  // the cells no earlier dim has taken
+                    lo = low_end(e);
+                    hi = std::max(G.n[e], lo);
+                } else if (e == d && side == 0) {
+                    hi = low_end(e);
+                } else if (e == d) {
+                    lo = std::max(G.n[e], low_end(e));
+                }
+                B.lo[b][e] = lo;
+                B.hi[b][e] = hi;
+                cells *= std::max(hi - lo, 0);
+            }
+            B.start[b] = total;
+            total += cells;
+        }
+    B.start[B.nbox] = total;
+    return B;
+}
+
+int64_t shell_blocks(const GhostShell& B) { return (B.start[B.nbox] + kT - 1) / kT; }
 
 int64_t blocks_of(const Range3& r)
 {
@@ -207,7 +263,7 @@ void launch_flux(int rs, const GridDev& G, const AdjRanges& R, const PerfectGas&
 int64_t adjoint_partials(const GridDev& G, int nd)
 {
     AdjRanges const R = adj_ranges(G, nd);
-    return blocks_of(R.ring1) + blocks_of(R.ring2) + blocks_of(R.flux);
+    return blocks_of(R.ring1) + blocks_of(R.ring2) + blocks_of(R.flux) + shell_blocks(adj_shell(G, nd));
 }
 
 #define HCLPP_ADJ_LIM_SWITCH(lim, BODY)                      \
@@ -239,17 +295,25 @@ int64_t launch_step_adjoint(int nd, int geom, int rs, int lim, const GridDev& G,
     // dgamma does not depend on how a run of reverse steps is split into calls.
     Range3 const& rg = R.ring2;
     int64_t off = 0;
+    bool const split = nd == 3 && R.interior.count() >= kSplitGather;
     HCLPP_ADJ_ND_SWITCH(nd, HCLPP_ADJ_GEOM_SWITCH(geom, {
-        if (!prims_ready) hipLaunchKernelGGL(k_adj_prim<ND>, range_grid(R.prim), blk, 0, s, G, R.prim, eos, A);
+        if (!prims_ready) hipLaunchKernelGGL(k_adj_prim<ND>, range_grid(R.ring2), blk, 0, s, G, R.ring2, eos, A);
         HCLPP_ADJ_LIM_SWITCH(lim, hipLaunchKernelGGL((k_adj_faces<ND, LIM, GEOM>), range_grid(R.ring1), blk, 0, s, G, R.ring1, eos, A,
                                                      partials, pending, dgamma));
         (launch_flux<ND, GEOM>)(rs, G, R, eos, A, partials, off, s);
         HCLPP_ADJ_LIM_SWITCH(lim, hipLaunchKernelGGL((k_adj_hancock<ND, LIM, GEOM>), range_grid(R.ring1), blk, 0, s, G, R.ring1, eos, A,
                                                      partials + off));
         off += blocks_of(R.ring1);
-        HCLPP_ADJ_LIM_SWITCH(lim, hipLaunchKernelGGL((k_adj_gather<ND, LIM>), range_grid(rg), blk, 0, s, G, rg, R.interior, eos, bc, A, nx,
-                                                     partials + off));
+        if (split)
+            hipLaunchKernelGGL((k_adj_gather<ND, false>), range_grid(rg), blk, 0, s, G, rg, R.interior, eos, bc, A, nx, partials + off);
+        else
+            hipLaunchKernelGGL((k_adj_gather<ND, true>), range_grid(rg), blk, 0, s, G, rg, R.interior, eos, bc, A, nx, partials + off);
         off += blocks_of(rg);
+        if (split) {
+            GhostShell const B = adj_shell(G, nd);
+            hipLaunchKernelGGL(k_adj_copies<ND>, dim3((unsigned)shell_blocks(B)), blk, 0, s, G, B, eos, bc, A, partials + off);
+            off += shell_blocks(B);
+        }
     }));
     if (!fold_now) return off;
     launch_adjoint_fold(partials, off, dgamma, s);

@@ -23,7 +23,8 @@
 //                               face-prim adjoints, the predictor's sources included), then of the
 //                               limited slopes: the cell's own prim adjoint and the shares owed to
 //                               its +-1 neighbours, overwriting the slots
-//   gather (interior cells)     cell-prim adjoint = own part + the neighbours' shares, prim -> cons
+//   gather (interior cells; the ghost part in a pass of its own on large grids)
+//                               cell-prim adjoint = own part + the neighbours' shares, prim -> cons
 //                               VJP, then the transposed ghost fill (every ghost cell whose value
 //                               was copied from this cell adds its adjoint back, sign-flipped where
 //                               the fill negated the momentum), the identity and gravity terms.
@@ -38,7 +39,6 @@
 namespace hclpp::adj {
 
 constexpr int kMaxGhosts = 4;
-constexpr int kMaxPre = 1 + 2 * kMaxGhosts;
 
 struct AdjArrays {
     const double* rho;  // step input, ghosts filled
@@ -505,50 +505,38 @@ __host__ __device__ __forceinline__ S<ND> cell_prim_adjoint(const GridDev& G, co
     return lp;
 }
 
-// Cells along dim d whose ghost-filled value is copied from interior index a (a itself first).
-__host__ __device__ __forceinline__ int preimages(const GridDev& G, const BcSpec& bc, int d, int a, int* pre, bool* flip)
+// Cells along one dim whose ghost-filled value is copied from interior index a: bit 0 a itself, then
+// the ng low ghosts, then the ng high ones; flip marks those whose normal momentum is negated.
+struct Copies {
+    unsigned cells, flip;
+};
+__host__ __device__ __forceinline__ Copies copies_of(const GridDev& G, const BcSpec& bc, int d, int a)
 {
-    int m = 0;
-    pre[m] = a;
-    flip[m] = false;
-    ++m;
+    Copies c{1u, 0u};
     int const ng = G.ngh[d], n = G.n[d], ext = G.nwg[d];
-    for (int g = 0; g < ng; ++g) {
+    for (int m = 1; m <= 2 * ng; ++m) {
         bool f = false;
-        if (face_map(bc.kind[2 * d], g, ng, n, ext, f) == a) {
-            pre[m] = g;
-            flip[m] = f;
-            ++m;
-        }
+        if (face_map(bc.kind[2 * d + (m > ng)], m <= ng ? m - 1 : n + m - 1, ng, n, ext, f) != a) continue;
+        c.cells |= 1u << m;
+        c.flip |= (unsigned)f << m;
     }
-    for (int g = ng + n; g < ext; ++g) {
-        bool f = false;
-        if (face_map(bc.kind[2 * d + 1], g, ng, n, ext, f) == a) {
-            pre[m] = g;
-            flip[m] = f;
-            ++m;
-        }
-    }
-    return m;
+    return c;
+}
+__host__ __device__ __forceinline__ int copy_cell(const GridDev& G, int d, int a, int m)
+{
+    return m == 0 ? a : (m <= G.ngh[d] ? m - 1 : G.n[d] + m - 1);
 }
 
-// Interior cells from which no ghost cell is filled, along dim d: [2 ng, n) in ghost-inclusive
-// indices (a periodic wrap fills the ghosts from [ng, 2 ng) and [n, n + ng), a Reflexive mirror
-// from the same cells, a NullGradient clamp from ng and ng + n - 1).
-__host__ __device__ __forceinline__ bool no_ghost_copies(const GridDev& G, int d, int lo, int hi)
-{
-    return lo >= 2 * G.ngh[d] && hi <= G.n[d];
-}
+// Whether some ghost cell may be filled from an interior index along dim d: the ng cells at either end
+// (a periodic wrap fills the ghosts from them, a Reflexive mirror too, a NullGradient clamp from the
+// outermost ones).
+__host__ __device__ __forceinline__ bool ghost_copies(const GridDev& G, int d, int a) { return a < 2 * G.ngh[d] || a >= G.n[d]; }
 
 // ---------------------------------------------------------------- pass 5: gather (interior cells)
-// DEEP: the cell is interior and no ghost is filled from it along any dim (no_ghost_copies), so
-// its only preimage is itself: the same sums in the same order as the general case, without the
-// preimage search.
-template <int ND, int LIM, bool DEEP = false>
-__host__ __device__ __forceinline__ double cell_gather(const GridDev& G, const PerfectGas& eos, const BcSpec& bc, const AdjArrays& A, int i,
-                                                       int j, int k)
+// The adjoint of cell (i, j, k) through the cell itself.
+template <int ND>
+__host__ __device__ __forceinline__ double gather_self(const GridDev& G, const PerfectGas& eos, const AdjArrays& A, int i, int j, int k)
 {
-    constexpr int NV = ND + 2;
     int64_t const pl = G.plane;
     int const c[3] = {i, j, k};
     int64_t const id = flat(G, i, j, k);
@@ -561,41 +549,47 @@ __host__ __device__ __forceinline__ double cell_gather(const GridDev& G, const P
         out[0] += A.dt * g * ln[1 + d];
         out[1 + d] += A.dt * g * ln[ND + 1];
     }
-    if constexpr (DEEP) {
-        double lg = 0;
-        S<ND> const lp = cell_prim_adjoint<ND, true>(G, A, c);
-        S<ND> lu = zero<ND>();
-        prim_vjp(load_cons<ND>(A.rho, A.rhou, A.E, id, pl), eos.gamma, lp, lu, lg);
-        out[0] += lu[0];
-#pragma unroll
-        for (int d = 0; d < ND; ++d) out[1 + d] += lu[1 + d];
-        out[ND + 1] += lu[ND + 1];
-        A.lrho[id] = out[0];
-#pragma unroll
-        for (int d = 0; d < ND; ++d) A.lrhou[id + pl * d] = out[1 + d];
-        A.lE[id] = out[ND + 1];
-        return lg;
-    }
-    int pre[3][kMaxPre];
-    bool flip[3][kMaxPre];
-    int npre[3] = {1, 1, 1};
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        pre[d][0] = c[d];
-        flip[d][0] = false;
-    }
-#pragma unroll
-    for (int d = 0; d < ND; ++d) npre[d] = preimages(G, bc, d, c[d], pre[d], flip[d]);
     double lg = 0;
-    for (int a = 0; a < npre[0]; ++a)
-        for (int b = 0; b < npre[1]; ++b)
-            for (int e = 0; e < npre[2]; ++e) {
-                int const q[3] = {pre[0][a], pre[1][b], pre[2][e]};
+    S<ND> const lp = cell_prim_adjoint<ND, true>(G, A, c);
+    S<ND> lu = zero<ND>();
+    prim_vjp(load_cons<ND>(A.rho, A.rhou, A.E, id, pl), eos.gamma, lp, lu, lg);
+    A.lrho[id] = out[0] + lu[0];
+#pragma unroll
+    for (int d = 0; d < ND; ++d) A.lrhou[id + pl * d] = out[1 + d] + lu[1 + d];
+    A.lE[id] = out[ND + 1] + lu[ND + 1];
+    return lg;
+}
+
+// Adds to the adjoint of cell (i, j, k) what reaches it through the ghost cells filled from it.
+template <int ND>
+__host__ __device__ __forceinline__ double gather_copies(const GridDev& G, const PerfectGas& eos, const BcSpec& bc, const AdjArrays& A, int i,
+                                                         int j, int k)
+{
+    int64_t const pl = G.plane;
+    int const c[3] = {i, j, k};
+    int64_t const id = flat(G, i, j, k);
+    Copies cp[3] = {{1u, 0u}, {1u, 0u}, {1u, 0u}};
+#pragma unroll
+    for (int d = 0; d < ND; ++d) cp[d] = copies_of(G, bc, d, c[d]);
+    if ((cp[0].cells | cp[1].cells | cp[2].cells) == 1u) return 0;
+    S<ND> out = load_cons<ND>(A.lrho, A.lrhou, A.lE, id, pl);
+    double lg = 0;
+    for (unsigned ma = cp[0].cells; ma; ma &= ma - 1)
+        for (unsigned mb = cp[1].cells; mb; mb &= mb - 1)
+            for (unsigned me = cp[2].cells; me; me &= me - 1) {
+                int const m[3] = {__builtin_ctz(ma), __builtin_ctz(mb), __builtin_ctz(me)};
+                if (m[0] + m[1] + m[2] == 0) continue;  // the cell itself
+                int q[3] = {c[0], c[1], c[2]};
+                bool fl[3] = {false, false, false};
+#pragma unroll
+                for (int d = 0; d < ND; ++d) {
+                    q[d] = copy_cell(G, d, c[d], m[d]);
+                    fl[d] = (cp[d].flip >> m[d]) & 1u;
+                }
                 S<ND> const lp = cell_prim_adjoint<ND>(G, A, q);
                 int64_t const qid = flat(G, q[0], q[1], q[2]);
                 S<ND> lu = zero<ND>();
                 prim_vjp(load_cons<ND>(A.rho, A.rhou, A.E, qid, pl), eos.gamma, lp, lu, lg);
-                bool const fl[3] = {flip[0][a], flip[1][b], flip[2][e]};
                 out[0] += lu[0];
 #pragma unroll
                 for (int d = 0; d < ND; ++d) out[1 + d] += fl[d] ? -lu[1 + d] : lu[1 + d];
@@ -606,6 +600,18 @@ __host__ __device__ __forceinline__ double cell_gather(const GridDev& G, const P
     for (int d = 0; d < ND; ++d) A.lrhou[id + pl * d] = out[1 + d];
     A.lE[id] = out[ND + 1];
     return lg;
+}
+
+template <int ND, int LIM>
+__host__ __device__ __forceinline__ double cell_gather(const GridDev& G, const PerfectGas& eos, const BcSpec& bc, const AdjArrays& A, int i,
+                                                       int j, int k)
+{
+    double const lg = gather_self<ND>(G, eos, A, i, j, k);
+    bool copies = false;
+    int const c[3] = {i, j, k};
+#pragma unroll
+    for (int d = 0; d < ND; ++d) copies = copies || ghost_copies(G, d, c[d]);
+    return copies ? lg + gather_copies<ND>(G, eos, bc, A, i, j, k) : lg;
 }
 
 }  // namespace hclpp::adj
