@@ -53,7 +53,6 @@ struct hclpp_ctx {
     int64_t fx_old_cap = 0;
     GhostShell shell{};
     MarchPlan march {};  // launch plan of the fused kernel
-    int march_occ = 0;    // its resident workgroups per CU
     int64_t fused_nb = 0;
     // passive scalars in a kernel of their own (scalars_apart): its plan, and the mass fluxes between
     // the two kernels (ndim planes of the storage type)
@@ -188,7 +187,7 @@ const DevFlag* clock_gate(const hclpp_ctx* c)
 }
 
 // Resident workgroups per CU of the fused kernel a context runs (without the fast arithmetic).
-int fused_occupancy(const hclpp_ctx* c)
+Residency fused_occupancy(const hclpp_ctx* c)
 {
     hclpp_config const& g = c->cfg;
     bool const f32 = g.precision == HCLPP_FP32_STORAGE;
@@ -397,12 +396,10 @@ int hclpp_ctx_create(const hclpp_config* cfg, hclpp_ctx** out)
         e = hipGetDevice(&dev);
         if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
         if (e != hipSuccess) return cleanup(hip_fail(e, "hipDeviceGetAttribute(multiProcessorCount)"));
-        int const occ = fused_occupancy(c);
-        c->march = plan_march(G, nd, occ, ncu);
-        c->march_occ = occ;
+        c->march = plan_march(G, nd, cfg->geom, fused_occupancy(c), ncu);
         if (c->scalars_apart) {
             bool const f32 = cfg->precision == HCLPP_FP32_STORAGE;
-            c->scalar_march = plan_march(G, nd, scalar_occupancy(nd, cfg->geom, cfg->limiter, cfg->nfx, f32), ncu);
+            c->scalar_march = plan_march(G, nd, cfg->geom, scalar_occupancy(nd, cfg->geom, cfg->limiter, cfg->nfx, f32), ncu);
             e = hipMalloc(&c->mflux, (f32 ? sizeof(float) : sizeof(double)) * G.plane * nd);
             if (e != hipSuccess) return cleanup(hip_fail(e, "hipMalloc(mass fluxes)"));
         }
@@ -834,14 +831,13 @@ int hclpp_set_pressure_fix(hclpp_ctx* c, int on, double eps)
 
 // Launch plan of the fused kernel the context runs (the plan depends on its occupancy) and the
 // partials buffer it fills.  Waits for the stream: the buffer may be reallocated.
-static int replan_march(hclpp_ctx* c, int occ)
+static int replan_march(hclpp_ctx* c, const Residency& occ)
 {
     int dev = 0, ncu = 0;
     HCLPP_HIP(hipGetDevice(&dev));
     HCLPP_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
     HCLPP_HIP(hipStreamSynchronize(c->stream));
-    c->march = plan_march(c->G, c->cfg.ndim, occ, ncu);
-    c->march_occ = occ;
+    c->march = plan_march(c->G, c->cfg.ndim, c->cfg.geom, occ, ncu);
     c->fused_nb = c->march.nb;
     return ensure_partials(c, c->fused_nb * kPartialStride);
 }
@@ -854,7 +850,7 @@ int hclpp_set_fast_arithmetic(hclpp_ctx* c, int on)
     if (on && c->pf_on) return fail(HCLPP_ERR_UNSUPPORTED, "the pressure fix runs with the reference arithmetic only");
     if ((on != 0) == (c->fast_on != 0)) return HCLPP_OK;
     int const nd = c->cfg.ndim;
-    int const occ = on ? march_occupancy_fast(nd, c->cfg.geom, c->cfg.riemann, c->cfg.limiter)
+    Residency const occ = on ? march_occupancy_fast(nd, c->cfg.geom, c->cfg.riemann, c->cfg.limiter)
                        : march_occupancy(nd, c->cfg.geom, c->cfg.riemann, c->cfg.limiter, false);
     int const rc = replan_march(c, occ);
     if (rc != HCLPP_OK) return rc;
@@ -1153,7 +1149,7 @@ int hclpp_fused_plan(hclpp_ctx* c, int* seglen, long long* workgroups, int* bloc
     if (!c || !seglen || !workgroups || !blocks_per_cu) return fail(HCLPP_ERR_ARG, "null argument");
     *seglen = c->march.L.seglen;
     *workgroups = c->march.nb;
-    *blocks_per_cu = c->march_occ;
+    *blocks_per_cu = c->march.per_cu;
     return HCLPP_OK;
 }
 

@@ -75,35 +75,47 @@ struct GhostShell {
     int64_t start[7];
 };
 
-// Workgroup shape of the fused kernel per dimensionality.
-template <int ND>
+// Workgroup shape of the march kernels per dimensionality; TALL: the second shape the 3D FP64 ones have.
+template <int ND, bool TALL = false>
 struct MarchShape;
-template <>
-struct MarchShape<1> {  // 64 independent segments per workgroup (plan_march sets their length)
+template <bool TALL>
+struct MarchShape<1, TALL> {  // 64 independent segments per workgroup (plan_march sets their length)
     static constexpr int HX = 1, HY = 1, NT = 64;
 };
-template <>
-struct MarchShape<2> {  // a 64-column row (62 outputs + halo) marching along y
+template <bool TALL>
+struct MarchShape<2, TALL> {  // a 64-column row (62 outputs + halo) marching along y
     static constexpr int HX = 64, HY = 1, NT = 64;
 };
 template <>
-struct MarchShape<3> {  // 16 x 16 columns (14 x 14 outputs + halo) marching along z
+struct MarchShape<3, false> {  // 16 x 16 columns (14 x 14 outputs + halo) marching along z
     // The halo columns repeat the predictor of their neighbours' faces: 16 x 16 computes 256
     // predictors for 196 outputs where 32 x 8 computed 256 for 180 (measured +11 % on RT 512^3).
     static constexpr int HX = 16, HY = 16, NT = 256;
+};
+template <>
+struct MarchShape<3, true> {  // 16 x 32 columns (14 x 30 outputs): 420 of 512, but one workgroup per CU
+    // whose barriers no other covers; plan_march says where it pays
+    static constexpr int HX = 16, HY = 32, NT = 512;
+};
+
+// Resident workgroups per CU of a march kernel in either shape (tall: 0 where it has no second one).
+struct Residency {
+    int normal, tall;
 };
 
 // Launch plan of the fused march kernel for one context.
 struct MarchPlan {
     FusedLayout L;
+    bool tall;   // the second shape
+    int per_cu;  // resident workgroups per CU of the shape taken
     int64_t nb;  // workgroups (one partials row each)
 };
-// Tile counts and segment length for a kernel of which blocks_per_cu workgroups are resident
-// per CU, on ncu CUs (see step_fused.hip for the cost model).
-MarchPlan plan_march(const GridDev& G, int nd, int blocks_per_cu, int ncu);
+// Shape, tile counts and segment length for a kernel of that residency on ncu CUs (see
+// step_fused.hip for the cost model).
+MarchPlan plan_march(const GridDev& G, int nd, int geom, const Residency& occ, int ncu);
 // Resident workgroups per CU of the k_step_march instance a configuration selects
 // without scalars (FP32 storage or not).
-int march_occupancy(int nd, int geom, int rs, int lim, bool fp32);
+Residency march_occupancy(int nd, int geom, int rs, int lim, bool fp32);
 void launch_fused_step(int nd, int geom, int rs, int lim, const GridDev& G, const MarchPlan& P, const PerfectGas& eos, const StepArrays& A,
                        hipStream_t s);
 void launch_fused_step(int nd, int geom, int rs, int lim, const GridDev& G, const MarchPlan& P, const PerfectGasMixed& eos,
@@ -111,25 +123,25 @@ void launch_fused_step(int nd, int geom, int rs, int lim, const GridDev& G, cons
 // the fused step with the opt-in fast FP64 arithmetic (step_fused_fast.hip; no passive scalars)
 void launch_fused_step(int nd, int geom, int rs, int lim, const GridDev& G, const MarchPlan& P, const PerfectGasFast& eos, const StepArrays& A,
                        hipStream_t s);
-int march_occupancy_fast(int nd, int geom, int rs, int lim);
+Residency march_occupancy_fast(int nd, int geom, int rs, int lim);
 // the fused step carrying one passive scalar (step_fused_fx.hip); A.fx and A.fx_new point at it
 void launch_fused_step_fx(int nd, int geom, int rs, int lim, const GridDev& G, const MarchPlan& P, const PerfectGas& eos, const StepArrays& A,
                           hipStream_t s);
 void launch_fused_step_fx(int nd, int geom, int rs, int lim, const GridDev& G, const MarchPlan& P, const PerfectGasMixed& eos,
                           const StepArraysF& A, hipStream_t s);
-int march_occupancy_fx(int nd, int geom, int rs, int lim, bool fp32);
+Residency march_occupancy_fx(int nd, int geom, int rs, int lim, bool fp32);
 // the fused step that stores the mass fluxes A.mflux (step_fused_mass.hip), and after it the passive
 // scalars A.nfx of them (step_scalars.hip), which read the mass fluxes and the new density
 void launch_fused_step_mass(int nd, int geom, int rs, int lim, const GridDev& G, const MarchPlan& P, const PerfectGas& eos, const StepArrays& A,
                             hipStream_t s);
 void launch_fused_step_mass(int nd, int geom, int rs, int lim, const GridDev& G, const MarchPlan& P, const PerfectGasMixed& eos,
                             const StepArraysF& A, hipStream_t s);
-int march_occupancy_mass(int nd, int geom, int rs, int lim, bool fp32);
+Residency march_occupancy_mass(int nd, int geom, int rs, int lim, bool fp32);
 int scalar_groups(int nfx);  // launches of the scalar kernel for nfx scalars
 void launch_scalar_march(int nd, int geom, int lim, const GridDev& G, const MarchPlan& P, const PerfectGas& eos, const StepArrays& A, hipStream_t s);
 void launch_scalar_march(int nd, int geom, int lim, const GridDev& G, const MarchPlan& P, const PerfectGasMixed& eos, const StepArraysF& A,
                          hipStream_t s);
-int scalar_occupancy(int nd, int geom, int lim, int nfx, bool fp32);
+Residency scalar_occupancy(int nd, int geom, int lim, int nfx, bool fp32);
 // the fused step's pressure fix (pressure_fix_fused.hip): after k_step_march, over the march
 // kernel's workgroups (plan P); fix_partials receives two doubles per workgroup
 void launch_pressure_fix_fused(int nd, int geom, int lim, const GridDev& G, const PerfectGas& eos, const StepArrays& A, const MarchPlan& P,

@@ -969,7 +969,12 @@ static void march_visit(int nd, int geom, int rs, int lim, V&& v)
 #undef HCLPP_FG
 }
 
-// Launch of k_step_march with the context's plan (tile counts, segment length, workgroups).
+// Whether a march kernel is built in the tall shape too: 3D with FP64 state (FP32 storage loses its
+// third wave per SIMD there: 256^3 12.5 -> 14.7 ms), without a carried scalar.
+template <class Eos, int ND, int NFX>
+constexpr bool kTallShape = ND == 3 && kFp64State<Eos> && NFX <= 0;
+
+// Launch of k_step_march with the context's plan (shape, tile counts, segment length, workgroups).
 template <class Eos, int NFX>
 struct MarchLaunch {
     const GridDev& G;
@@ -977,29 +982,45 @@ struct MarchLaunch {
     const Eos& eos;
     const StepArraysT<typename Eos::real>& A;
     hipStream_t s;
-    template <int ND, int GEOM, int RS, int LIM>
-    void run() const
+    template <int ND, int GEOM, int RS, int LIM, bool TALL>
+    void launch() const
     {
-        using S = MarchShape<ND>;
-        if (P.nb == 0) return;
+        using S = MarchShape<ND, TALL>;
         hipLaunchKernelGGL((k_step_march<Eos, ND, GEOM, RS, LIM, NFX, S::HX, S::HY, S::NT>), dim3((unsigned)P.nb), dim3(S::NT), 0, s, G, eos,
                            A, P.L);
     }
+    template <int ND, int GEOM, int RS, int LIM>
+    void run() const
+    {
+        if (P.nb == 0) return;
+        if constexpr (kTallShape<Eos, ND, NFX>) {
+            if (P.tall) return launch<ND, GEOM, RS, LIM, true>();
+        }
+        launch<ND, GEOM, RS, LIM, false>();
+    }
 };
 
-// Resident workgroups per CU of one k_step_march instance (its registers and LDS decide).
+// Resident workgroups per CU of a kernel of nt threads (its registers and LDS decide).
+template <class K>
+static int resident(K kernel, int nt)
+{
+    int n = 0;
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, nt, 0) == hipSuccess ? n : 0;
+}
+
 template <class Eos, int NFX>
 struct MarchOccupancy {
-    int* out;
+    Residency* out;
     template <int ND, int GEOM, int RS, int LIM>
     void run() const
     {
         using S = MarchShape<ND>;
-        int n = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_step_march<Eos, ND, GEOM, RS, LIM, NFX, S::HX, S::HY, S::NT>, S::NT, 0) !=
-            hipSuccess)
-            n = 0;
-        *out = n;
+        out->normal = resident(k_step_march<Eos, ND, GEOM, RS, LIM, NFX, S::HX, S::HY, S::NT>, S::NT);
+        out->tall = 0;
+        if constexpr (kTallShape<Eos, ND, NFX>) {
+            using T = MarchShape<ND, true>;
+            out->tall = resident(k_step_march<Eos, ND, GEOM, RS, LIM, NFX, T::HX, T::HY, T::NT>, T::NT);
+        }
     }
 };
 

@@ -119,14 +119,20 @@ struct FixLaunch {
     const MarchPlan& P;
     double* partials;
     hipStream_t s;
+    template <int ND, int GEOM, int LIM, bool TALL>
+    void launch() const
+    {
+        using S = MarchShape<ND, TALL>;
+        hipLaunchKernelGGL((k_pressure_fix_fused<ND, GEOM, LIM, S::HX, S::HY, S::NT>), dim3((unsigned)P.nb), dim3(S::NT), 0, s, G, eos, A, P.L,
+                           partials);
+    }
     template <int ND, int GEOM, int RS, int LIM>
     void run() const
     {
-        using S = MarchShape<ND>;
         if constexpr (RS == kHLL) {  // the fix does not depend on the Riemann solver: one instance per limiter
             if (P.nb == 0) return;
-            hipLaunchKernelGGL((k_pressure_fix_fused<ND, GEOM, LIM, S::HX, S::HY, S::NT>), dim3((unsigned)P.nb), dim3(S::NT), 0, s, G, eos,
-                               A, P.L, partials);
+            if (P.tall) launch<ND, GEOM, LIM, true>();
+            else launch<ND, GEOM, LIM, false>();
         }
     }
 };

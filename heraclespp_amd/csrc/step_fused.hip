@@ -198,23 +198,31 @@ __global__ __launch_bounds__(1024) void k_clock_advance(DevClock* c, const doubl
 //   44.4 us with 4, 32.8 with 2 (one wave per SIMD), 37.0 with 1 (two waves).
 // The split changes which workgroup computes a cell, not how: results do not depend on it (the
 // conserved totals, summed per workgroup, only change their summation order).
-MarchPlan plan_march(const GridDev& G, int nd, int blocks_per_cu, int ncu)
+//
+// The 3D FP64 kernels have a second, tall shape (16 x 32 columns) whose tiles waste less on halo rows,
+// 30 outputs of 32 against 14 of 16, but whose single workgroup per CU leaves its barriers uncovered:
+// at equal tile counts it takes 2 % longer (Cartesian 251 x 190 x 133 and 512^3) to 9 % (spherical 512 x
+// 128 x 256). It is taken where its plan's cost is lower by more than that: spherical 160 x 60 x 60
+// with five scalars 3.80 -> 2.95 ms, 96 x 200 x 64 1.96 -> 1.75; 50 x 41 x 37 would go 1.74 -> 2.20.
+static MarchPlan plan_shape(const GridDev& G, int nd, bool tall, int blocks_per_cu, int ncu, int64_t& best_cost)
 {
     MarchPlan P{};
+    P.tall = tall;
+    P.per_cu = blocks_per_cu;
     int const nm = G.n[nd - 1];
     int const TX = nd == 1 ? 1 : (nd == 2 ? MarchShape<2>::HX : MarchShape<3>::HX) - 2;
-    int const TY = nd == 3 ? MarchShape<3>::HY - 2 : 1;
+    int const TY = nd == 3 ? (tall ? MarchShape<3, true>::HY : MarchShape<3>::HY) - 2 : 1;
     P.L.ntile[0] = nd == 1 ? 1 : (G.n[0] + TX - 1) / TX;
     P.L.ntile[1] = nd == 3 ? (G.n[1] + TY - 1) / TY : 1;
     int64_t const tiles = (int64_t)P.L.ntile[0] * P.L.ntile[1];
     int64_t const cus = std::max(ncu, 1), per_cu = std::max(blocks_per_cu, 1);
     int64_t const resident = per_cu * cus;
-    int const waves = (nd == 1 ? MarchShape<1>::NT : nd == 2 ? MarchShape<2>::NT : MarchShape<3>::NT) / 64;
+    int const waves = (nd == 1 ? MarchShape<1>::NT : nd == 2 ? MarchShape<2>::NT : tall ? MarchShape<3, true>::NT : MarchShape<3>::NT) / 64;
     auto plane_cost = [&](int64_t blocks) -> int64_t {  // 4 c(w) with `blocks` workgroups spread over the chip
         int64_t const w = ((blocks + cus - 1) / cus * waves + 3) / 4;  // four SIMDs per CU
         return w > 0 ? 4 * w + 1 : 0;
     };
-    int64_t best_cost = -1;
+    best_cost = -1;
     for (int seg = std::min(1, nm); seg <= std::min(nm, 1 << 16); ++seg) {
         int64_t const segs = (nm + seg - 1) / seg;
         // 1D: a workgroup holds one segment per thread
@@ -229,9 +237,18 @@ MarchPlan plan_march(const GridDev& G, int nd, int blocks_per_cu, int ncu)
     return P;
 }
 
-int march_occupancy(int nd, int geom, int rs, int lim, bool fp32)
+MarchPlan plan_march(const GridDev& G, int nd, int geom, const Residency& occ, int ncu)
 {
-    int n = 0;
+    int64_t cost = 0, cost_tall = 0;
+    MarchPlan const P = plan_shape(G, nd, false, occ.normal, ncu, cost);
+    if (occ.tall <= 0) return P;
+    MarchPlan const T = plan_shape(G, nd, true, occ.tall, ncu, cost_tall);
+    return cost_tall * (geom == kSpherical ? 112 : 106) < cost * 100 ? T : P;
+}
+
+Residency march_occupancy(int nd, int geom, int rs, int lim, bool fp32)
+{
+    Residency n{};
     if (fp32) march_visit(nd, geom, rs, lim, MarchOccupancy<PerfectGasMixed, 0>{&n});
     else march_visit(nd, geom, rs, lim, MarchOccupancy<PerfectGas, 0>{&n});
     return n;

@@ -14,9 +14,9 @@ void launch_fused_step(int nd, int geom, int rs, int lim, const GridDev& G, cons
     march_visit(nd, geom, rs, lim, MarchLaunch<PerfectGasFast, 0>{G, P, eos, A, s});
 }
 
-int march_occupancy_fast(int nd, int geom, int rs, int lim)
+Residency march_occupancy_fast(int nd, int geom, int rs, int lim)
 {
-    int n = 0;
+    Residency n{};
     march_visit(nd, geom, rs, lim, MarchOccupancy<PerfectGasFast, 0>{&n});
     return n;
 }

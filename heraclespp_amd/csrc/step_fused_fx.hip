@@ -22,9 +22,9 @@ void launch_fused_step_fx(int nd, int geom, int rs, int lim, const GridDev& G, c
     march_visit(nd, geom, rs, lim, MarchLaunch<PerfectGasMixed, 1>{G, P, eos, A, s});
 }
 
-int march_occupancy_fx(int nd, int geom, int rs, int lim, bool fp32)
+Residency march_occupancy_fx(int nd, int geom, int rs, int lim, bool fp32)
 {
-    int n = 0;
+    Residency n{};
     if (fp32) march_visit(nd, geom, rs, lim, MarchOccupancy<PerfectGasMixed, 1>{&n});
     else march_visit(nd, geom, rs, lim, MarchOccupancy<PerfectGas, 1>{&n});
     return n;

@@ -19,9 +19,9 @@ void launch_fused_step_mass(int nd, int geom, int rs, int lim, const GridDev& G,
     march_visit(nd, geom, rs, lim, MarchLaunch<PerfectGasMixed, kStoreMass>{G, P, eos, A, s});
 }
 
-int march_occupancy_mass(int nd, int geom, int rs, int lim, bool fp32)
+Residency march_occupancy_mass(int nd, int geom, int rs, int lim, bool fp32)
 {
-    int n = 0;
+    Residency n{};
     if (fp32) march_visit(nd, geom, rs, lim, MarchOccupancy<PerfectGasMixed, kStoreMass>{&n});
     else march_visit(nd, geom, rs, lim, MarchOccupancy<PerfectGas, kStoreMass>{&n});
     return n;

@@ -42,25 +42,35 @@ struct ScalarLaunch {
     const MarchPlan& P;
     const StepArraysT<typename Eos::real>& A;
     hipStream_t s;
+    template <int ND, int GEOM, int LIM, int NF, bool TALL>
+    void launch() const
+    {
+        using S = MarchShape<ND, TALL>;
+        hipLaunchKernelGGL((k_scalar_march<Eos, ND, GEOM, LIM, NF, S::HX, S::HY, S::NT>), dim3((unsigned)P.nb), dim3(S::NT), 0, s, G, A, P.L);
+    }
     template <int ND, int GEOM, int LIM, int NF>
     void run() const
     {
-        using S = MarchShape<ND>;
-        hipLaunchKernelGGL((k_scalar_march<Eos, ND, GEOM, LIM, NF, S::HX, S::HY, S::NT>), dim3((unsigned)P.nb), dim3(S::NT), 0, s, G, A, P.L);
+        if constexpr (kTallShape<Eos, ND, 0>) {
+            if (P.tall) return launch<ND, GEOM, LIM, NF, true>();
+        }
+        launch<ND, GEOM, LIM, NF, false>();
     }
 };
 
 template <class Eos>
 struct ScalarOccupancy {
-    int* out;
+    Residency* out;
     template <int ND, int GEOM, int LIM, int NF>
     void run() const
     {
         using S = MarchShape<ND>;
-        int n = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_scalar_march<Eos, ND, GEOM, LIM, NF, S::HX, S::HY, S::NT>, S::NT, 0) != hipSuccess)
-            n = 0;
-        *out = n;
+        out->normal = resident(k_scalar_march<Eos, ND, GEOM, LIM, NF, S::HX, S::HY, S::NT>, S::NT);
+        out->tall = 0;
+        if constexpr (kTallShape<Eos, ND, 0>) {
+            using T = MarchShape<ND, true>;
+            out->tall = resident(k_scalar_march<Eos, ND, GEOM, LIM, NF, T::HX, T::HY, T::NT>, T::NT);
+        }
     }
 };
 
@@ -93,11 +103,11 @@ void launch_scalar_march(int nd, int geom, int lim, const GridDev& G, const Marc
     launch_scalars_any<PerfectGasMixed>(nd, geom, lim, G, P, A, s);
 }
 
-int scalar_occupancy(int nd, int geom, int lim, int nfx, bool fp32)
+Residency scalar_occupancy(int nd, int geom, int lim, int nfx, bool fp32)
 {
     int const groups = scalar_groups(nfx);
     int const nf = (nfx + groups - 1) / groups;  // the largest group
-    int n = 0;
+    Residency n{};
     if (fp32) scalar_visit(nd, geom, lim, nf, ScalarOccupancy<PerfectGasMixed>{&n});
     else scalar_visit(nd, geom, lim, nf, ScalarOccupancy<PerfectGas>{&n});
     return n;
