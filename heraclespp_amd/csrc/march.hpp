@@ -138,14 +138,23 @@ __device__ __forceinline__ double state_eint(const Eos& eos, const State<ND, typ
 }
 
 // The distances of a cell's center to its neighbours' along one dim, with their reciprocals
-// (GridDev::hc): (dx[i-1] + dx[i]) / 2 and (dx[i] + dx[i+1]) / 2.
+// (GridDev::hc): (dx[i-1] + dx[i]) / 2 and (dx[i] + dx[i+1]) / 2.  With FP32 state the distances are FP32
+// sums and the reciprocals v_rcp_f32's, as PerfectGasMixed::div takes them: rounding the table's
+// instead moves a blast wave's far field by 1e-5.
 struct CenterDist {
     double hm, ym, hp, yp;
 };
+template <class Eos>
 __device__ __forceinline__ CenterDist center_dist(const GridDev& G, int dim, int i)
 {
-    double const* h = G.hc[dim] + 2 * (i - 1);
-    return {h[0], h[1], h[2], h[3]};
+    if constexpr (kFp64State<Eos>) {
+        double const* h = G.hc[dim] + 2 * (i - 1);
+        return {h[0], h[1], h[2], h[3]};
+    } else {
+        float const dl = (float)G.dx[dim][i];
+        float const hm = ((float)G.dx[dim][i - 1] + dl) * 0.5f, hp = (dl + (float)G.dx[dim][i + 1]) * 0.5f;
+        return {hm, __builtin_amdgcn_rcpf(hm), hp, __builtin_amdgcn_rcpf(hp)};
+    }
 }
 
 // limited_linear_reconstruction.hpp:53-62 for one variable along one dim
@@ -225,7 +234,7 @@ __device__ __forceinline__ void predict_faces(const GridDev& G, const Eos& eos, 
 #pragma unroll
     for (int dim = 0; dim < ND; ++dim) {
         T const dl = T(G.dx[dim][idx[dim]]);
-        CenterDist const h = center_dist(G, dim, idx[dim]);
+        CenterDist const h = center_dist<Eos>(G, dim, idx[dim]);
 #pragma unroll
         for (int v = 0; v < NV; ++v)
             reconstruct<LIM, Eos>(nb[dim][0][v], p[v], nb[dim][1][v], h, dl, fp[0][dim][v], fp[1][dim][v]);

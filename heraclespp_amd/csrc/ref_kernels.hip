@@ -153,7 +153,7 @@ __global__ __launch_bounds__(256) void k_muscl_hancock(GridDev G, Range3 r, Perf
 #pragma unroll
     for (int dim = 0; dim < ND; ++dim) {
         double const dl = G.dx[dim][idx[dim]];
-        CenterDist const h = center_dist(G, dim, idx[dim]);
+        CenterDist const h = center_dist<PerfectGas>(G, dim, idx[dim]);
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             double const* q = prim_plane(v) + id;
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(256) void k_muscl_hancock(GridDev G, Range3 r, Perf
         double xo[2][ND], d[ND];
 #pragma unroll
         for (int dim = 0; dim < ND; ++dim) {
-            CenterDist const h = center_dist(G, dim, idx[dim]);
+            CenterDist const h = center_dist<PerfectGas>(G, dim, idx[dim]);
             reconstruct<LIM, PerfectGas>(q[-stride[dim]], q[0], q[stride[dim]], h, G.dx[dim][idx[dim]], xo[0][dim], xo[1][dim]);
             double const dS = face_area<ND, GEOM>(G, dim, i, j, k);
             double const dSp = face_area<ND, GEOM>(G, dim, i + (dim == 0), j + (dim == 1), k + (dim == 2));

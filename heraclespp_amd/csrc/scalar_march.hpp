@@ -169,7 +169,7 @@ __global__ __launch_bounds__(NT, ND == 3 ? 2 : 1) void k_scalar_march(GridDev G,
         T dl[ND];
 #pragma unroll
         for (int d = 0; d < ND; ++d) {
-            hd[d] = center_dist(G, d, idx[d]);
+            hd[d] = center_dist<Eos>(G, d, idx[d]);
             dl[d] = T(G.dx[d][idx[d]]);
             dS[d] = T(face_area<ND, GEOM>(G, d, ci, cj, ck));
             dSp[d] = T(face_area<ND, GEOM>(G, d, ci + (d == 0), cj + (d == 1), ck + (d == 2)));
