@@ -245,7 +245,8 @@ int hclpp_step(hclpp_ctx* ctx, const double* rho, const double* rhou, const doub
  * state (hydro_reconstruction.hpp:99-109), carried through the Hancock half step as a partial
  * density (extrapolation_reconstruction.hpp:87-88, 105-108, 315-337), upwinded with the mass
  * flux and clamped to [0, 1] in the update (godunov_scheme.hpp:122, 263-301).  One scalar
- * is carried by the hydro kernel; several follow it in a kernel of their own, four per launch. */
+ * is carried by the hydro kernel (in 3D FP64 Cartesian, below 2^21 cells); otherwise they follow it
+ * in a kernel of their own, four per launch, and the context holds ndim planes of mass fluxes. */
 int hclpp_step_fx(hclpp_ctx* ctx, const double* rho, const double* rhou, const double* E, const double* fx, double* rho_new,
                   double* rhou_new, double* E_new, double* fx_new);
 
