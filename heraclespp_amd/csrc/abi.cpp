@@ -53,11 +53,12 @@ struct hclpp_ctx {
     int64_t fx_old_cap = 0;
     GhostShell shell{};
     MarchPlan march {};  // launch plan of the fused kernel
-    int64_t fused_nb = 0;
     // passive scalars in a kernel of their own (scalars_apart): its plan, and the mass fluxes between
-    // the two kernels (ndim planes of the storage type)
+    // the two kernels (ndim planes of the storage type, reserve_mflux); a step without them takes the
+    // kernel that carries a scalar, once per scalar, by its own plan
     bool scalars_apart = false;
     MarchPlan scalar_march {};
+    MarchPlan carried_march {};
     void* mflux = nullptr;
     double* gtab = nullptr;         // radial gravity table (inside tables; rebuilt for internal-mass gravity)
     double* shells = nullptr;       // internal-mass gravity: per-layer sums of rho dV and dV
@@ -194,6 +195,25 @@ Residency fused_occupancy(const hclpp_ctx* c)
     if (g.nfx == 0) return march_occupancy(g.ndim, g.geom, g.riemann, g.limiter, f32);
     if (c->scalars_apart) return march_occupancy_mass(g.ndim, g.geom, g.riemann, g.limiter, f32);
     return march_occupancy_fx(g.ndim, g.geom, g.riemann, g.limiter, f32);
+}
+
+// Launch plan of the hydro kernel that the next step takes, and the workgroups (partials rows) of the
+// largest plan a step of the context may take.
+const MarchPlan& step_plan(const hclpp_ctx* c) { return c->scalars_apart && !c->mflux ? c->carried_march : c->march; }
+int64_t step_blocks(const hclpp_ctx* c) { return std::max(c->march.nb, c->carried_march.nb); }
+
+// The mass fluxes between the two kernels of a step with scalars apart, taken when a clock starts:
+// no step allocates, and contexts that only run operators hold none.  Where the device lacks the
+// memory (with a gibibyte to spare, for the kernels' scratch) the steps carry the scalars instead.
+void reserve_mflux(hclpp_ctx* c)
+{
+    if (!c->scalars_apart || c->mflux) return;
+    size_t const bytes = (c->cfg.precision == HCLPP_FP32_STORAGE ? sizeof(float) : sizeof(double)) * (size_t)c->G.plane * c->cfg.ndim;
+    size_t const spare = (size_t)1 << 30;
+    size_t available = 0, total = 0;
+    if (hipMemGetInfo(&available, &total) == hipSuccess && available >= bytes + spare && hipMalloc(&c->mflux, bytes) == hipSuccess) return;
+    c->mflux = nullptr;
+    (void)hipGetLastError();  // not the next launch's error
 }
 
 int read_scalar(hclpp_ctx* c, double* out)
@@ -400,17 +420,15 @@ int hclpp_ctx_create(const hclpp_config* cfg, hclpp_ctx** out)
         if (c->scalars_apart) {
             bool const f32 = cfg->precision == HCLPP_FP32_STORAGE;
             c->scalar_march = plan_march(G, nd, cfg->geom, scalar_occupancy(nd, cfg->geom, cfg->limiter, cfg->nfx, f32), ncu);
-            e = hipMalloc(&c->mflux, (f32 ? sizeof(float) : sizeof(double)) * G.plane * nd);
-            if (e != hipSuccess) return cleanup(hip_fail(e, "hipMalloc(mass fluxes)"));
+            c->carried_march = plan_march(G, nd, cfg->geom, march_occupancy_fx(nd, cfg->geom, cfg->riemann, cfg->limiter, f32), ncu);
         }
     }
-    c->fused_nb = c->march.nb;
     Range3 all;
     for (int d = 0; d < 3; ++d) {
         all.b[d] = 0;
         all.e[d] = G.nwg[d];
     }
-    int64_t const need = std::max<int64_t>(c->fused_nb * kPartialStride, reduce_blocks(all));
+    int64_t const need = std::max<int64_t>(step_blocks(c) * kPartialStride, reduce_blocks(all));
     int const rc = ensure_partials(c, need);
     if (rc != HCLPP_OK) return cleanup(rc);
     *out = c;
@@ -718,20 +736,28 @@ static int fused_step(hclpp_ctx* c, const S* rho, const S* rhou, const S* E, con
     }
     bool const timed = c->prof_count < c->prof_max;
     if (timed) HCLPP_HIP(hipEventRecord(c->prof_events[2 * c->prof_count], c->stream));
-    if (nfx > 0 && c->scalars_apart) {
+    MarchPlan const& plan = step_plan(c);
+    if (nfx > 0 && c->scalars_apart && c->mflux) {
         // the scalars are upwinded with the hydro step's mass fluxes (godunov_scheme.hpp:263-301) and
         // do not act on it: the hydro kernel stores those, and the scalar kernel follows
-        launch_fused_step_mass(nd, c->cfg.geom, c->cfg.riemann, c->cfg.limiter, c->G, c->march, eos, A, c->stream);
+        launch_fused_step_mass(nd, c->cfg.geom, c->cfg.riemann, c->cfg.limiter, c->G, plan, eos, A, c->stream);
         launch_scalar_march(nd, c->cfg.geom, c->cfg.limiter, c->G, c->scalar_march, eos, A, c->stream);
     } else if (nfx > 0) {
-        launch_fused_step_fx(nd, c->cfg.geom, c->cfg.riemann, c->cfg.limiter, c->G, c->march, eos, A, c->stream);
+        // each launch writes the same hydro update and partials, and its own scalar
+        for (int f = 0; f < nfx; ++f) {
+            StepArraysT<S> Af = A;
+            Af.fx = fx + c->G.plane * f;
+            Af.fx_new = fx_new + c->G.plane * f;
+            Af.nfx = 1;
+            launch_fused_step_fx(nd, c->cfg.geom, c->cfg.riemann, c->cfg.limiter, c->G, plan, eos, Af, c->stream);
+        }
     } else {
         bool fast = false;
         if constexpr (!f32) fast = c->fast_on;
         if constexpr (!f32) {
-            if (fast) launch_fused_step(nd, c->cfg.geom, c->cfg.riemann, c->cfg.limiter, c->G, c->march, c->eos_fast, A, c->stream);
+            if (fast) launch_fused_step(nd, c->cfg.geom, c->cfg.riemann, c->cfg.limiter, c->G, plan, c->eos_fast, A, c->stream);
         }
-        if (!fast) launch_fused_step(nd, c->cfg.geom, c->cfg.riemann, c->cfg.limiter, c->G, c->march, eos, A, c->stream);
+        if (!fast) launch_fused_step(nd, c->cfg.geom, c->cfg.riemann, c->cfg.limiter, c->G, plan, eos, A, c->stream);
     }
     HCLPP_LAUNCHED("fused step");
     if (timed) {
@@ -740,14 +766,14 @@ static int fused_step(hclpp_ctx* c, const S* rho, const S* rhou, const S* E, con
     }
     if constexpr (!f32) {
         if (c->pf_on) {  // main.cpp:459-475: after the update, before the boundaries
-            launch_pressure_fix_fused(nd, c->cfg.geom, c->cfg.limiter, c->G, eos, A, c->march, c->fix_partials, c->stream);
+            launch_pressure_fix_fused(nd, c->cfg.geom, c->cfg.limiter, c->G, eos, A, plan, c->fix_partials, c->stream);
             HCLPP_LAUNCHED("pressure fix (fused step)");
         }
     }
     launch_ghosts_rate(nd, c->cfg.geom, c->G, eos, c->bc, c->shell, A, c->stream);
     HCLPP_LAUNCHED("ghost fill");
-    launch_clock_advance(nd, c->clock, c->partials, c->fused_nb, c->ghost_partials, c->ghost_cap, c->pf_on && !f32 ? c->fix_partials : nullptr,
-                         c->pf_on && !f32 ? c->fix_nb : 0, c->stream);
+    launch_clock_advance(nd, c->clock, c->partials, plan.nb, c->ghost_partials, c->ghost_cap, c->pf_on && !f32 ? c->fix_partials : nullptr,
+                         c->pf_on && !f32 ? plan.nb : 0, c->stream);
     HCLPP_LAUNCHED("clock advance");
     return HCLPP_OK;
 }
@@ -787,6 +813,7 @@ static int clock_reset(hclpp_ctx* c, double t0, int iter0, double t_end, double 
     if (c->cfg.ng < 2) return fail(HCLPP_ERR_ARG, "the fused step needs ng >= 2 (two-cell reconstruction stencil)");
     DevClock* h = c->host_clock;
     HCLPP_HIP(hipStreamSynchronize(c->stream));  // the pinned staging buffer is reused
+    reserve_mflux(c);
     std::memset(h, 0, sizeof(DevClock));
     h->pub.t = t0;
     h->pub.iter = iter0;
@@ -814,13 +841,13 @@ int hclpp_set_pressure_fix(hclpp_ctx* c, int on, double eps)
     if (on && c->cfg.precision != HCLPP_FP64) return fail(HCLPP_ERR_UNSUPPORTED, "the pressure fix runs with FP64 storage only");
     if (on && c->fast_on) return fail(HCLPP_ERR_UNSUPPORTED, "the pressure fix runs with the reference arithmetic only");
     if (on && !std::isfinite(eps)) return fail(HCLPP_ERR_ARG, "eps must be finite");
-    if (on && (!c->fix_partials || c->fix_nb != c->fused_nb)) {  // one pair per workgroup of the march kernel's plan
+    if (on && (!c->fix_partials || c->fix_nb < step_blocks(c))) {  // one pair per workgroup of the march kernel's plan
         if (c->fix_partials) {
             HCLPP_HIP(hipStreamSynchronize(c->stream));
             HCLPP_HIP(hipFree(c->fix_partials));
             c->fix_partials = nullptr;
         }
-        int64_t const nb = c->fused_nb;
+        int64_t const nb = step_blocks(c);
         HCLPP_HIP(hipMalloc(&c->fix_partials, sizeof(double) * 2 * (nb > 0 ? nb : 1)));
         c->fix_nb = nb;
     }
@@ -838,8 +865,7 @@ static int replan_march(hclpp_ctx* c, const Residency& occ)
     HCLPP_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
     HCLPP_HIP(hipStreamSynchronize(c->stream));
     c->march = plan_march(c->G, c->cfg.ndim, c->cfg.geom, occ, ncu);
-    c->fused_nb = c->march.nb;
-    return ensure_partials(c, c->fused_nb * kPartialStride);
+    return ensure_partials(c, c->march.nb * kPartialStride);
 }
 
 int hclpp_set_fast_arithmetic(hclpp_ctx* c, int on)
@@ -883,6 +909,7 @@ static int clock_resume_reset(hclpp_ctx* c)
     HCLPP_HIP(hipStreamSynchronize(c->stream));
     if (h->pub.status) return fail(HCLPP_ERR_STATE, "the clock stopped on an error");
     if (h->pub.exiting) return fail(HCLPP_ERR_ARG, "the run has ended (t_end or max_iter reached)");
+    reserve_mflux(c);
     h->pub.done = 0;
     h->pub.output_due = 0;
     h->pending_exit = 0;

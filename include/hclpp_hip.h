@@ -246,7 +246,9 @@ int hclpp_step(hclpp_ctx* ctx, const double* rho, const double* rhou, const doub
  * density (extrapolation_reconstruction.hpp:87-88, 105-108, 315-337), upwinded with the mass
  * flux and clamped to [0, 1] in the update (godunov_scheme.hpp:122, 263-301).  One scalar
  * is carried by the hydro kernel (in 3D FP64 Cartesian, below 2^21 cells); otherwise they follow it
- * in a kernel of their own, four per launch, and the context holds ndim planes of mass fluxes. */
+ * in a kernel of their own, four per launch, and the context holds ndim planes of mass fluxes from its
+ * first clock start on.  Where the device has no memory for those, the hydro kernel runs once per
+ * scalar instead, with the same results. */
 int hclpp_step_fx(hclpp_ctx* ctx, const double* rho, const double* rhou, const double* E, const double* fx, double* rho_new,
                   double* rhou_new, double* E_new, double* fx_new);
 
