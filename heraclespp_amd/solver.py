@@ -39,6 +39,11 @@ def _dev(a, shape, device="cuda"):
     return a
 
 
+def _overlap(a, b) -> bool:
+    """Whether two contiguous tensors share memory."""
+    return a.data_ptr() < b.data_ptr() + b.nbytes and b.data_ptr() < a.data_ptr() + a.nbytes
+
+
 class HydroSolver:
     def __init__(self, grid: Grid, eos: PerfectGas, *, reconstruction: str = "VanLeer", riemann_solver: str = "HLL",
                  gravity=None, bc=None, bc_order=None, cfl: float = 0.4, nfx: int = 0, fused: bool = True,
@@ -134,6 +139,8 @@ class HydroSolver:
         rho_d, u_d, P_d = _dev(rho, g.shape3), _dev(u, (nd,) + g.shape3), _dev(P, g.shape3)
         self._cur = 0
         r, m, E = self._cons[0]
+        # u and P are read in place, after rho is written: what is given in the state's own arrays is copied first
+        u_d, P_d = (t.clone() if any(_overlap(t, s) for s in (r, m, E)) else t for t in (u_d, P_d))
         r.copy_(rho_d)
         if self.nfx:
             self.fx.copy_(_dev(fx, (self.nfx,) + g.shape3))
