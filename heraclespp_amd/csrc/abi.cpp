@@ -400,7 +400,9 @@ int hclpp_ctx_create(const hclpp_config* cfg, hclpp_ctx** out)
     // fills the chip).  Runs of 10 steps on MI355X, carried / apart: one scalar 2D 2048^2 3.08 / 3.82 ms,
     // 3D spherical 160 x 60 x 60 1.85 / 2.35, FP32 128^3 2.10 / 2.51, FP64 50 x 41 x 37 0.69 / 0.74,
     // 128^3 4.18 / 4.12, 250^3 26.0 / 23.5; two (a hydro kernel per scalar / apart) 2D 2048^2 5.57 / 4.10,
-    // 250^3 49.7 / 25.5, 160 x 60 x 60 3.33 / 2.49.
+    // 250^3 49.7 / 25.5, 160 x 60 x 60 3.33 / 2.49.  Around the line, microseconds a step: 64^3 101 / 105,
+    // 112^3 242 / 251, 128^3 414 / 420, 144^3 575 / 575, 160^3 747 / 733, 256^3 2868 / 2729; where a last round
+    // of workgroups falls matters as much (120^3 327 / 312, 400 x 60 x 80 395 / 343, 60 x 400 x 100 496 / 506).
     c->scalars_apart = cfg->nfx >= 2
                        || (cfg->nfx == 1 && nd == 3 && cfg->geom == HCLPP_GEOM_CARTESIAN && cfg->precision == HCLPP_FP64
                            && (int64_t)G.n[0] * G.n[1] * G.n[2] >= (int64_t)1 << 21);

@@ -1,8 +1,10 @@
 // adjoint.hip -- reverse-mode hydro step on gfx950 (Cartesian or spherical geometry, HLL/HLLC,
 // every limiter, uniform or point-mass gravity, every boundary kind), dt held fixed.
 //
-// Five passes over 64 x 4 workgroups (x fastest, coalesced SoA planes); each output element
-// is written by exactly one thread, and the dL/dgamma contributions are reduced per
+// Five passes whose workgroups walk each plane's cells in memory order where that pays
+// (in_memory_order; 64 x 4 blocks of x and y elsewhere), and on large 3D grids a sixth over the cells
+// that ghosts are filled from (k_adj_copies, which adds to what the gather wrote).  Each pass writes
+// an output element by exactly one thread, and the dL/dgamma contributions are reduced per
 // workgroup and folded in a fixed order, so the gradient is bit-reproducible run to run.
 // In a run of reverse steps, each step's gather pass also forms the primitives the next one
 // needs, so the primitive pass runs once per run, and each step's faces pass folds the

@@ -602,6 +602,7 @@ __host__ __device__ __forceinline__ double gather_copies(const GridDev& G, const
     return lg;
 }
 
+// Both, as one pass takes them.  LIM is the passes' common parameter: the gather is the same for every limiter.
 template <int ND, int LIM>
 __host__ __device__ __forceinline__ double cell_gather(const GridDev& G, const PerfectGas& eos, const BcSpec& bc, const AdjArrays& A, int i,
                                                        int j, int k)

@@ -80,10 +80,12 @@ __host__ __device__ __forceinline__ double fdiv(double a, double b)
 #endif
 }
 
-// Quotients that share a divisor.  recip(b) is fdiv's reciprocal, recip_near(b, y0) the same from
-// a y0 already within a few ulp of 1 / b (the last of fdiv's two Newton steps squares that error,
-// far below an ulp, so both end at the same double) and quot(a, b, y) the rest of fdiv:
-// bit-identical to fdiv(a, b) on its range.  v_rcp_f64 issues in 16.6 cycles on MI355X where an
+// Quotients that share a divisor.  recip(b) is fdiv's reciprocal, recip_near(b, y0) one step from a
+// y0 already within a few ulp of 1 / b, and quot(a, b, y) the rest of fdiv: with recip's y bit-identical
+// to fdiv(a, b) on its range.  A Newton step squares the error of its start, so recip_near rounds a
+// value within 2^-98 of 1 / b, as recip does; that the two land on one double for every b is not proven,
+// nor that quot would always correct a last bit: tests/cpp/quot_check finds no quotient that differs
+// from IEEE division among 2^22 pairs of each form.  v_rcp_f64 issues in 16.6 cycles on MI355X where an
 // FP64 fma takes 4.8 (measured), so a reciprocal from scratch costs 7.5 fma and one from a
 // neighbour (1 / (rho kb) from 1 / rho) three; one that depends on the grid or the equation of
 // state alone is read from a table or a kernel argument.

@@ -14,8 +14,11 @@
 
 namespace hclpp {
 
-// STREAM: a store that bypasses the caches, for outputs larger than the last-level cache (conversions
-// of 512^3 5 to 8 % faster, 320^3 2 to 5 %).
+// STREAM: a store that bypasses the caches, for outputs larger than the last-level cache.  Conversions,
+// cached / streaming: 512^3 5 to 8 % faster, 320^3 2 to 5 %, 224^3 (361 MB of outputs) 3 %, 200^3 (259 MB)
+// and 2D 3300^2 (249 MB) equal.  Below it a conversion on its own gains as well (176^3 76 / 62 us), but what
+// reads its outputs next finds them in the cache: with a pass over them 176^3 takes 129 / 135 us, 128^3
+// 53 / 56, 2D 2600^2 108 / 118, 200^3 200 / 204, 224^3 285 / 283.
 template <bool STREAM>
 __device__ __forceinline__ void put(double& to, double v)
 {

@@ -69,7 +69,7 @@ __global__ __launch_bounds__(NT, ND == 3 ? 2 : 1) void k_scalar_march(GridDev G,
     int const ring_a = ND >= 2 ? min(mc.ox - 2 + ring_px, G.nwg[0] - 1) : 0;
     int const ring_b = ND == 3 ? min(mc.oy - 2 + ring_py, G.nwg[1] - 1) : 0;
 
-    // density and velocities of a cell (NU components), as the conversion of its state forms them
+    // density and momenta of a cell or, once divided, its velocities, as the conversion of its state forms them
     struct Q {
         T rho, m[ND];
     };

@@ -202,8 +202,12 @@ __global__ __launch_bounds__(1024) void k_clock_advance(DevClock* c, const doubl
 // The 3D FP64 kernels have a second, tall shape (16 x 32 columns) whose tiles waste less on halo rows,
 // 30 outputs of 32 against 14 of 16, but whose single workgroup per CU leaves its barriers uncovered:
 // at equal tile counts it takes 2 % longer (Cartesian 251 x 190 x 133 and 512^3) to 9 % (spherical 512 x
-// 128 x 256). It is taken where its plan's cost is lower by more than that: spherical 160 x 60 x 60
-// with five scalars 3.80 -> 2.95 ms, 96 x 200 x 64 1.96 -> 1.75; 50 x 41 x 37 would go 1.74 -> 2.20.
+// 128 x 256): spherical 160 x 60 x 60 with five scalars 3.80 -> 2.95 ms, 96 x 200 x 64 1.96 -> 1.75, but
+// 50 x 41 x 37 would go 1.74 -> 2.20.  The cost model does not know that loss, so plan_march asks for a
+// margin.  Both shapes on 80 grids of 0.2 to 8 M cells (normal / tall kernel time by normal / tall cost):
+// Cartesian 0.94 to 1.14 at cost ratios from 0.98 to 1.03, 1.03 and more from 1.06 on; spherical 0.92 to
+// 1.20 at ratios from 0.98 to 1.05, 1.04 to 1.08 from there to 1.105, 1.07 and more from 1.11 on.  The lines,
+// 1.06 and 1.12, lie where no grid measured loses.
 static MarchPlan plan_shape(const GridDev& G, int nd, bool tall, int blocks_per_cu, int ncu, int64_t& best_cost)
 {
     MarchPlan P{};
