@@ -39,11 +39,6 @@ def _dev(a, shape, device="cuda"):
     return a
 
 
-def _overlap(a, b) -> bool:
-    """Whether two contiguous tensors share memory."""
-    return a.data_ptr() < b.data_ptr() + b.nbytes and b.data_ptr() < a.data_ptr() + a.nbytes
-
-
 class HydroSolver:
     def __init__(self, grid: Grid, eos: PerfectGas, *, reconstruction: str = "VanLeer", riemann_solver: str = "HLL",
                  gravity=None, bc=None, bc_order=None, cfl: float = 0.4, nfx: int = 0, fused: bool = True,
@@ -140,7 +135,11 @@ class HydroSolver:
         self._cur = 0
         r, m, E = self._cons[0]
         # u and P are read in place, after rho is written: what is given in the state's own arrays is copied first
-        u_d, P_d = (t.clone() if any(_overlap(t, s) for s in (r, m, E)) else t for t in (u_d, P_d))
+        at_r, at_m, at_E, at_u, at_P, plane = r.data_ptr(), m.data_ptr(), E.data_ptr(), u_d.data_ptr(), P_d.data_ptr(), 8 * r.numel()
+        if -nd * plane < at_u - at_r < plane or -nd * plane < at_u - at_m < nd * plane or -nd * plane < at_u - at_E < plane:
+            u_d = u_d.clone()
+        if -plane < at_P - at_r < plane or -plane < at_P - at_m < nd * plane or -plane < at_P - at_E < plane:
+            P_d = P_d.clone()
         r.copy_(rho_d)
         if self.nfx:
             self.fx.copy_(_dev(fx, (self.nfx,) + g.shape3))
