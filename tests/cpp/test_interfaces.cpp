@@ -371,8 +371,8 @@ static void test_passive_scalar_loop(int const nfx)
             hu[c] = band ? 0.5 : -0.5;
             hu[c + cells] = 0.01 * std::sin(4 * M_PI * x) * std::sin(5.0 * x + 2.0 * y);
             hP[c] = 2.5;
-            // scalar 0 traces the band, 1 its complement, 2 a smooth field (nfx > 1: one fused
-            // launch per scalar)
+            // scalar 0 traces the band, 1 its complement, 2 a smooth field (nfx > 1: the scalar kernel
+            // after the hydro one)
             for (int f = 0; f < nfx; ++f)
                 hfx[c + cells * f] = f == 0 ? (band ? 1.0 : 0.0) : f == 1 ? (band ? 0.0 : 1.0) : 0.5 + 0.4 * std::sin(2 * M_PI * (x + f * y));
         }

@@ -64,8 +64,8 @@ def test_gpu_reverse_step_matches_host_build(cuda, case):
     assert abs(gpu[3] - host[3]) <= 1e-12 * max(1.0, abs(host[3]))
 
 
-# Grids wide enough for the gather pass's workgroups (64 x 4 cells) to lie where no ghost copies
-# from, which take the gather without the preimage search; the host build searches every cell.
+# Grids wide enough that most waves of the gather pass hold no cell that a ghost is filled from (and
+# below the size from which 3D grids leave the ghosts' part to a pass of its own).
 LARGE_CASES = [
     ("2d_large_vanalbada_hllc_mixed_g", 2, [160, 24], "VanAlbada", "HLLC", ["Periodic", "Periodic", "Reflexive", "NullGradient"],
      (0.0, -0.2, 0)),

@@ -1,7 +1,7 @@
 """Several passive scalars on the fused step (hclpp_step_fx with nfx > 1), against the oracle.
 
-The fused kernel carries one scalar per launch; with nfx scalars the step launches it nfx times,
-the first launch also writing the hydro update and the CFL/totals partials.  Each scalar is
+The hydro kernel stores the mass flux through every face, and a kernel of their own then carries the
+scalars, up to four per launch.  Each scalar is
 reconstructed, extrapolated as a partial density and upwinded with the same mass flux
 (extrapolation_reconstruction.hpp:87-88, 105-108, 315-337; godunov_scheme.hpp:263-301), so every
 array must equal the oracle's, bit for bit, the clock included.
@@ -67,7 +67,7 @@ def test_fused_step_several_scalars_match_oracle(cuda, name):
 
 
 def test_identical_scalars_stay_identical(cuda):
-    """Three copies of one field: each launch computes the same scalar update, so the three planes
+    """Three copies of one field: the scalar kernel computes the same update for each, so the three planes
     are equal, and equal to the one-scalar step's plane."""
     s = setups.kelvin_helmholtz(32, seed=2)
     y = (s.rho > 1.5).astype(np.float64)

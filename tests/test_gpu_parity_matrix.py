@@ -69,7 +69,7 @@ def _oracle(s, kw, fx=None):
 def test_step_matches_oracle_bitwise(cuda, nd, geom, lim, rs, path):
     """fused: hclpp_step; operators: the reference kernel sequence (hclpp_hydro_reconstruction,
     hclpp_godunov, ...); fused_2_scalars: hclpp_step_fx with two seeded passive scalars (mass
-    fractions in [0, 1]), one launch per scalar."""
+    fractions in [0, 1]), carried by the scalar kernel after the hydro one."""
     s, kw = _case(nd, geom, lim, rs)
     fx = None
     if path == "fused_2_scalars":

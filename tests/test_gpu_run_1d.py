@@ -62,8 +62,8 @@ def test_one_launch_is_the_steps_one_by_one(cuda, n, geom, ng, riemann, limiter,
 
 
 def test_t_end_and_the_discarded_step(cuda):
-    """A run that ends inside a batch at t_end, and one whose state turns invalid: the state, the count
-    and the time are those of the steps that were completed."""
+    """A run that ends inside a batch at t_end, and one whose first step finds an invalid state: the state,
+    the count and the time are those of the steps that were completed."""
     for kill in (False, True):
         sols = [_solver(300, "Cartesian", 2, "HLLC", "VanLeer", "fp64", ["Periodic", "Periodic"]) for _ in range(2)]
         init = _initial(sols[0].grid, 1)

@@ -1,5 +1,5 @@
 """The march kernels' second tile shape (16 x 32 columns, 3D FP64) against the oracle, bit for bit, on
-grids whose launch plan takes it: a last tile row that is full, one row over, ragged; scalars and the
+grids whose launch plan takes it: a last tile row that is full or ragged; scalars and the
 pressure fix in it; and the fast arithmetic."""
 
 import ctypes
