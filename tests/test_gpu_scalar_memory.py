@@ -83,11 +83,14 @@ def test_steps_without_memory_for_the_mass_fluxes(cuda):
     planes = 3 * 8 * (n + 4) ** 3
     state = 2 * 7 * 8 * (n + 4) ** 3
     filler = torch.empty(_free() - state - planes, dtype=torch.uint8, device="cuda")
-    print(f"[scalar memory] {filler.numel() >> 20} MiB set aside, {_free() >> 20} MiB free", flush=True)
-    took, _ = _run(n, steps, save)
-    assert not took
-    del filler, save
-    _free()
+    try:
+        print(f"[scalar memory] {filler.numel() >> 20} MiB set aside, {_free() >> 20} MiB free", flush=True)
+        took, _ = _run(n, steps, save)
+        assert not took
+    finally:
+        filler.untyped_storage().resize_(0)  # also where a failure's traceback holds the tensor
+        del save
+        _free()
 
 
 def test_steps_captured_before_the_clock_starts(cuda):
